@@ -31,6 +31,12 @@ HIP_FLAGS = [
 ]
 
 
+# Flags of single sources.  gdn2_fwd.hip: the scan kernels hold their operands in
+# up to 512 registers; results of matrix instructions stay in vector registers
+# (the default above 256 is accumulation registers, and a copy for every use).
+SOURCE_FLAGS = {"gdn2_fwd.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
+
+
 def hipcc() -> str:
     for cand in (os.environ.get("HIPCC"), shutil.which("hipcc"), "/opt/rocm/bin/hipcc"):
         if cand and Path(cand).exists():
@@ -41,7 +47,7 @@ def hipcc() -> str:
 def _compile(src: str, verbose: bool) -> Path:
     obj = BUILD / (Path(src).stem + ".o")
     lang = ["-x", "hip"]
-    cmd = [hipcc(), *HIP_FLAGS, *lang, f"-I{CSRC}", f"-I{ROOT / 'include'}", "-c",
+    cmd = [hipcc(), *HIP_FLAGS, *SOURCE_FLAGS.get(src, []), *lang, f"-I{CSRC}", f"-I{ROOT / 'include'}", "-c",
            str(CSRC / src), "-o", str(obj)]
     if verbose:
         print(" ".join(cmd), flush=True)

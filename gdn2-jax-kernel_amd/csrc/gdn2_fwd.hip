@@ -28,6 +28,7 @@
 
 #include "gdn2_common.h"
 #include "gdn2_layout.h"
+#include "gdn2_scan.h"
 #include "gdn2_stage.h"
 
 namespace gdn2 {
@@ -41,7 +42,8 @@ struct PrepArgs {
   int T_len, H, N;
   long long NC;   // number of chunks, B*H*N
   float scale;
-  T* W;     // [cid][BT][D]; float32: in the split pair layout (kPrepFull)
+  T* W;     // [cid][BT][D]; kPrepFull: bfloat16 -W in fragment order (gdn2_scan.h),
+            // float32 W in the split pair layout
   T* UT;
   T* KgT;   // [cid][D][BT]; float32: in the split pair layout (kPrepFull)
   T* Qg;
@@ -483,7 +485,7 @@ __global__ void __launch_bounds__(64 * prep_waves(BT), prep_min_blocks(sizeof(T)
           if constexpr (SPF) {
             split_store1(reinterpret_cast<char*>(kgT + (size_t)(d0 + ch) * BT), t, kgv);
           } else if constexpr (MODE == kPrepFull) {
-            kgT[(size_t)(d0 + ch) * BT + kpos<T>(t)] = from_f<T>(kgv);
+            kgT[frag_off<BT>(d0 + ch, t)] = from_f<T>(kgv);
           }
           kgr[e] = kgv;
           kh[e] = kv * ekh;
@@ -499,8 +501,20 @@ __global__ void __launch_bounds__(64 * prep_waves(BT), prep_min_blocks(sizeof(T)
           dk[e] = kv * edk;
         }
         if constexpr (MODE != kPrepScores)
-          *reinterpret_cast<Op*>(a.frag ? qgf + qg_frag<T, BT, D>(I, d0 / KS + j, lane)
-                                        : qgp + j * KS + lg * KC) = op_from<T>(qg);
+        {
+          const Op qv = op_from<T>(qg);
+          if (!a.frag) {
+            *reinterpret_cast<Op*>(qgp + j * KS + lg * KC) = qv;
+          } else if constexpr (sizeof(T) == 4) {
+            *reinterpret_cast<Op*>(qgf + qg_frag<T, BT, D>(I, d0 / KS + j, lane)) = qv;
+          } else {
+            // chained order: this lane's eight channels 8 lg + e belong to the lane
+            // groups 2 (lg % 2) and 2 (lg % 2) + 1, half lg / 2
+            T* f = qgf + frag_off<D>(t, d0 + j * KS + lg * KC);
+            *reinterpret_cast<bf16x4*>(f) = __builtin_shufflevector(qv, qv, 0, 1, 2, 3);
+            *reinterpret_cast<bf16x4*>(f + 128) = __builtin_shufflevector(qv, qv, 4, 5, 6, 7);
+          }
+        }
         if constexpr (MODE == kPrepWy) {   // kg [t][d]
           *reinterpret_cast<Op*>(a.KgT + (size_t)cid * BT * D + (size_t)t * D + d0 + j * KS +
                                  lg * KC) = op_from<T>(kgr);
@@ -827,15 +841,19 @@ __global__ void __launch_bounds__(64 * prep_waves(BT), prep_min_blocks(sizeof(T)
       if constexpr (SPF) {
         split_store4(reinterpret_cast<char*>(Wc + (size_t)(I * 16 + li) * D), dg + 4 * lg,
                      sanitize4(accw));
+      } else if constexpr (sizeof(T) == 4) {
+        store4(Wc + (size_t)(I * 16 + li) * D + dg + 4 * lg, sanitize4(accw));
       } else {
-        store4(Wc + (size_t)(I * 16 + li) * D + kpos<T>(dg + 4 * lg), sanitize4(accw));
+        store4(Wc + frag_off<D>(I * 16 + li, dg + 4 * lg), -sanitize4(accw));
       }
       if constexpr (MODE == kPrepWy) {   // u [t][d]
         T* uc = a.UT + (size_t)cid * BT * D;
 #pragma unroll
         for (int r = 0; r < 4; ++r) uc[(size_t)(I * 16 + 4 * lg + r) * D + dg + li] = sanitize(accu[r]);
+      } else if constexpr (sizeof(T) == 4) {
+        store4(Uc + (size_t)(dg + li) * BT + I * 16 + 4 * lg, sanitize4(accu));
       } else {
-        store4(Uc + (size_t)(dg + li) * BT + kpos<T>(I * 16 + 4 * lg), sanitize4(accu));
+        store4(Uc + frag_off<BT>(dg + li, I * 16 + 4 * lg), sanitize4(accu));
       }
     }
   }
@@ -1669,22 +1687,40 @@ __global__ void __launch_bounds__(256) seg_combine(const float* seg, const float
   }
   __syncthreads();
   bool bound = false;   // a clip of an entry state bound (see StateArgs::sat)
-  for (int s = 1; s + 1 < S; ++s) {
+  // M and e of a step do not depend on the state: loaded one segment ahead
+  constexpr int NJ = (NDT + 3) / 4;
+  f32x4 mn[NJ][NDT], en[NJ];
+  auto load_seg = [&](int s) __attribute__((always_inline)) {
     const float* M = segb + ((size_t)s * 2 + 1) * DD;
     const float* e = segb + (size_t)s * 2 * DD;
-    f32x4 acc[(NDT + 3) / 4];
 #pragma unroll
-    for (int j = 0; j < (NDT + 3) / 4; ++j) {
+    for (int j = 0; j < NJ; ++j) {
       const int at = wv + 4 * j;
-      acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
       if (at < NDT) {
 #pragma unroll
         for (int kt = 0; kt < NDT; ++kt)
-          mma(acc[j], load4f(M + (size_t)(at * 16 + li) * D + kt * 16 + 4 * lg),
-              load4f(&sHT[li * (D + 4) + kt * 16 + 4 * lg]));
+          mn[j][kt] = load4f(M + (size_t)(at * 16 + li) * D + kt * 16 + 4 * lg);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) en[j][r] = e[(size_t)(at * 16 + 4 * lg + r) * D + c0 + li];
       }
     }
-    __syncthreads();  // every wave has read the current state
+  };
+  if (S > 2) load_seg(1);
+  for (int s = 1; s + 1 < S; ++s) {
+    f32x4 acc[NJ], e[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const int at = wv + 4 * j;
+      acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      e[j] = en[j];
+      if (at < NDT) {
+#pragma unroll
+        for (int kt = 0; kt < NDT; ++kt)
+          mma(acc[j], mn[j][kt], load4f(&sHT[li * (D + 4) + kt * 16 + 4 * lg]));
+      }
+    }
+    if (s + 2 < S) load_seg(s + 1);
+    lds_barrier();  // every wave has read the current state
 #pragma unroll
     for (int j = 0; j < (NDT + 3) / 4; ++j) {
       const int at = wv + 4 * j;
@@ -1694,7 +1730,7 @@ __global__ void __launch_bounds__(256) seg_combine(const float* seg, const float
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const size_t o = (size_t)(at * 16 + 4 * lg + r) * D + c0 + li;
-          const float x = acc[j][r] + e[o];
+          const float x = acc[j][r] + e[j][r];
           bound = bound || !(fabsf(x) <= g_clip);
           nh[r] = sanitize(x);
           hinb[(size_t)(s + 1) * DD + o] = nh[r];
@@ -1702,7 +1738,7 @@ __global__ void __launch_bounds__(256) seg_combine(const float* seg, const float
         store4(&sHT[li * (D + 4) + at * 16 + 4 * lg], nh);
       }
     }
-    __syncthreads();
+    lds_barrier();
   }
   if (__ballot(bound) != 0 && lane == 0) *sat = 1;
 }
@@ -1832,6 +1868,32 @@ __global__ void __launch_bounds__(256) fwd_out(OutArgs<T> a) {
 }
 
 // ---------------------------------------------------------------------------
+// One scan launch: `units` (b,h) pairs, times segments or sequences; `outputs`
+// with output waves.  Column slices of 16 while they all fit the device at one
+// workgroup per CU (the shortest step: 0.8 us a chunk of 64 at D = 128, bfloat16,
+// against 1.1 with 32 columns), else of 32 (each loaded operand then feeds two
+// products: 48 (b,h) of 128 such chunks take 195 us against 280 with 16).
+template <typename T, int BT, int D>
+void launch_scan(hipStream_t st, ScanArgs<T> a, size_t units, bool outputs) {
+  constexpr int KS = scan_ksplit(sizeof(T), D);
+  const int sm = a.summary ? 2 : 1;
+  a.units = (int)units;
+  if (units == 0) return;
+  auto go = [&](auto cpc) {
+    constexpr int CPW = decltype(cpc)::value, NVS = D / (16 * CPW);
+    constexpr int NO = scan_out_waves(sizeof(T), KS, CPW);
+    const dim3 grid(scan_grid(units, NVS * sm));
+    if (outputs)
+      hipLaunchKernelGGL((fwd_scan<T, BT, D, KS, CPW, NO>), grid, dim3(64 * (KS + NO + 1)), 0,
+                         st, a);
+    else
+      hipLaunchKernelGGL((fwd_scan<T, BT, D, KS, CPW, 0>), grid, dim3(64 * (KS + 1)), 0, st, a);
+  };
+  if (units * sm * (D / 16) <= 256) go(std::integral_constant<int, 1>{});
+  else go(std::integral_constant<int, 2>{});
+}
+
+// ---------------------------------------------------------------------------
 // Host launchers (called from gdn2_api.cpp).
 template <typename T, typename TG, int BT, int D, typename TI>
 hipError_t launch_fwd(hipStream_t st, int B, int T_len, int H, const void* q, const void* k,
@@ -1843,7 +1905,7 @@ hipError_t launch_fwd(hipStream_t st, int B, int T_len, int H, const void* q, co
   // the segment count follows flags only (the workspace was sized from them): the
   // final pass of an inference forward is the 32-column scan with output waves
   constexpr int NO = state_out_waves<T, BT, D>();
-  const bool fuse_ws = NO > 0 && !(flags & 1);
+  const bool fuse_ws = scan_outputs(sizeof(T), D) && !(flags & 1);
   const int S_ws = vl ? 1
                       : state_segments((long long)B * H, N, D, (int)sizeof(T), (flags >> 8) & 0xff,
                                        fuse_ws ? 32 : seg_pass_cols(sizeof(T), D));
@@ -1877,6 +1939,55 @@ hipError_t launch_fwd(hipStream_t st, int B, int T_len, int H, const void* q, co
                        pa);
   }
   launch_mark(st);
+  if constexpr (sizeof(T) == 2) {
+    const size_t BH = (size_t)B * H;
+    ScanArgs<T> sa{};
+    sa.W = W;
+    sa.UT = UT;
+    sa.KgT = KgT;
+    sa.GL = GL;
+    sa.h0 = h0;
+    sa.N = N;
+    sa.S = 1;
+    sa.L = N;
+    sa.HT = HT;
+    sa.VnT = VnT;
+    sa.h_final = h_final;
+    sa.H = H;
+    sa.Qg = Qg;
+    sa.Aqk = Aqk;
+    sa.out = out;
+    sa.scale = scale;
+    sa.T_len = T_len;
+    if (vl) {   // one unit per (head, sequence)
+      sa.cu = vl->cu_chunks;
+      sa.cstart = vl->cstart;
+      sa.S = vl->nseq;
+      launch_scan<T, BT, D>(st, sa, BH * vl->nseq, fuse);
+    } else if (S_ws > 1) {
+      float* seg = reinterpret_cast<float*>(ws + L.SEG);            // [bh][S][2][D][D]
+      float* hin = seg + BH * S_ws * 2 * (size_t)D * D;              // [bh][S][D][D]
+      ScanArgs<T> pa = sa;
+      pa.S = S_ws;
+      pa.L = (N + S_ws - 1) / S_ws;
+      pa.sat = sat;
+      pa.summary = 1;
+      pa.seg = seg;
+      launch_scan<T, BT, D>(st, pa, BH * S_ws, false);
+      hipLaunchKernelGGL((seg_combine<D>), dim3(BH * (D / 16)), dim3(256), 0, st, seg, h0, hin,
+                         S_ws, sat);
+      pa.summary = 0;
+      pa.hin = hin;
+      launch_scan<T, BT, D>(st, pa, BH * S_ws, fuse);
+      // A clip of the state bound somewhere in the segmented passes: the segments'
+      // affine combination does not hold, and the serial scan recomputes everything
+      // the final pass wrote; otherwise its workgroups return at once
+      sa.gate = sat;
+      launch_scan<T, BT, D>(st, sa, BH, fuse);
+    } else {
+      launch_scan<T, BT, D>(st, sa, BH, fuse);
+    }
+  } else {
   constexpr int SW = 2;  // compute waves (16 value columns each) per state workgroup
   constexpr int SP = 4;  // producer waves (DMA issue: 4 beat 2 by 14 % on float32 scans)
   constexpr int SK = state_ksplit<T, BT, D>();   // compute waves per column slice
@@ -1943,6 +2054,7 @@ hipError_t launch_fwd(hipStream_t st, int B, int T_len, int H, const void* q, co
     else
       hipLaunchKernelGGL((fwd_state<T, BT, D, SW, SP, SK>), dim3(BH * NVS), dim3(NTH), 0, st,
                          sa);
+  }
   }
   launch_mark(st);
   if (NC > 0 && !fuse) {

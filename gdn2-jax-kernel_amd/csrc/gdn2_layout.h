@@ -191,6 +191,18 @@ constexpr int state_out_waves_of(int esize, int BT, int D) {
           lds <= 160 * 1024) ? BT / 32 : 0;
 }
 
+// The forward scan (fwd_scan in gdn2_scan.h): whether an inference scan forms the
+// outputs itself (then no h^T / v_new^T tiles exist), here so that the host's
+// workspace size follows the same choice; its state waves per column slice (what
+// keeps a wave's operands in its registers) and its output waves.
+constexpr bool scan_outputs(int esize, int D) { return esize == 2 || D == 64; }
+constexpr int scan_ksplit(int esize, int D) {
+  return esize == 2 ? (D > 128 ? 2 : 1) : (D >= 256 ? 4 : 2);
+}
+constexpr int scan_out_waves(int esize, int ksplit, int cpw) {
+  return esize == 4 ? 4 : (ksplit == 1 && cpw == 1 ? 2 : 1);
+}
+
 // Segments of the forward state scan for BH (b,h) pairs of N chunks with
 // `esize`-byte tiles, whose final pass runs workgroups of `final_cols` value
 // columns (seg_pass_cols, or 32 for the inference scan with output waves).

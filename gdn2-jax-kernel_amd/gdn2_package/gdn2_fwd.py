@@ -281,16 +281,18 @@ def _residual_views(p: _Prepared, ws: torch.Tensor):
     shp = (B, H, N)
     idx = torch.arange(BT, device=p.device)
     causal = (idx[:, None] >= idx[None, :])
-    # bfloat16 W, UT, KgT, HT, VnT keep their last dimension in chained order
-    # (gdn2_common.h kpos): undo it for the views
+    # bfloat16 HT, VnT keep their last dimension in chained order (gdn2_common.h
+    # kpos); W (stored negated), UT, KgT are in operand-fragment order
+    # (gdn2_scan.h): undo it
     chained = p.tile_dt == torch.bfloat16
     nat = lambda x, n: x[..., _kpos_index(n, x.device)] if chained else x
     # float32 W and KgT are in the scans' split pair layout: decode them
-    spl = (lambda x: x) if chained else _split_decode
+    tile = lambda x: _frag_decode(x) if chained else x
+    spl = _frag_decode if chained else _split_decode
     return {
-        "w_pseudo": f(spl(nat(views["W"].view(*shp, BT, D), D))),
-        "u": f(nat(views["UT"].view(*shp, D, BT), BT).transpose(-1, -2)),
-        "kg": f(spl(nat(views["KgT"].view(*shp, D, BT), BT)).transpose(-1, -2)),
+        "w_pseudo": f(spl(views["W"].view(*shp, BT, D))) * (-1.0 if chained else 1.0),
+        "u": f(tile(views["UT"].view(*shp, D, BT)).transpose(-1, -2)),
+        "kg": f(spl(views["KgT"].view(*shp, D, BT)).transpose(-1, -2)),
         "qg": f(views["Qg"].view(*shp, BT, D)),
         "Aqk": torch.where(causal, f(views["Aqk"].view(*shp, BT, BT)), 0.0),
         "gc_last": f(views["GL"].view(*shp, D)),
@@ -308,6 +310,16 @@ def _split_decode(x: torch.Tensor) -> torch.Tensor:
     parts = x.contiguous().view(torch.bfloat16).reshape(*lead, L // 32, 2, 4, 2, 4).float()
     val = parts[..., 0, :, :, :] + parts[..., 1, :, :, :]          # (.., runs, j, half, slot)
     return val.transpose(-3, -2).reshape(*lead, L)                  # element 16 half + 4 j + slot
+
+
+def _frag_decode(x: torch.Tensor) -> torch.Tensor:
+    """Tiles (..., R, K) stored in operand-fragment order (csrc/gdn2_scan.h
+    frag_off) in natural order: fragment (row tile, 32-deep k-group), lane 16 lg + li
+    = row li, its eight elements k = 16 half + 4 lg + r at 4 half + r."""
+    *lead, R, K = x.shape
+    y = x.contiguous().view(*lead, R // 16, K // 32, 4, 16, 2, 4)   # rt, kk, lg, li, half, r
+    n = len(lead)
+    return y.permute(*range(n), n, n + 3, n + 1, n + 4, n + 2, n + 5).reshape(*lead, R, K)
 
 
 def _kpos_index(n: int, device) -> torch.Tensor:
