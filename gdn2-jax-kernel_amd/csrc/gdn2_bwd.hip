@@ -15,6 +15,7 @@
 
 #include "gdn2_common.h"
 #include "gdn2_layout.h"
+#include "gdn2_scan.h"
 #include "gdn2_stage.h"
 
 namespace gdn2 {
@@ -99,6 +100,10 @@ __device__ __forceinline__ void stage_store(float* dst, int ld, const Staged& s,
 // ============================================================================
 // bwd_state (B1): reverse scan over chunks; workgroup = (b,h, 32 value columns of dh).
 // ============================================================================
+template <int D>
+hipError_t launch_bwd_scan(hipStream_t st, size_t nchunks, const float* W, const float* KgT,
+                           float* kg, float* wt, BScanArgs a);   // gdn2_fwd.hip
+
 template <typename T>
 struct BStateArgs {
   const T* W;        // [cid][BT][D]
@@ -2210,8 +2215,32 @@ hipError_t launch_bwd_wide(hipStream_t st, int B, int T_len, int H, const void* 
                    dh_final, N, buf(B_DHT), buf(B_DVNT), dh0, cu_chunks, cu_chunks ? nseq : 1, H};
   constexpr int BW = 2, BK = bstate_ksplit<T, D>(), BP = BK > 1 ? 4 : 2;
   const size_t units = cu_chunks ? (size_t)H * nseq : (size_t)B * H;
-  hipLaunchKernelGGL((bwd_state<T, BT, D, BW, BP, BK>), dim3(units * (D / (16 * BW))),
-                     dim3(64 * (BW * BK + BP)), 0, st, sa);
+  // B1: where the units leave CUs free, the scan over fragment tiles (the transposed
+  // tiles go into the DQG / DKG regions, which B3 writes afterwards); else bwd_state
+  bool frag = false;
+  if constexpr (sizeof(T) == 4) {
+    frag = !scan_rows(4, units, D);
+    if (frag) {
+      BScanArgs fa{};
+      fa.GL = sa.GL;
+      fa.DVPT = sa.DVPT;
+      fa.QDOT = sa.QDOT;
+      fa.dh_final = dh_final;
+      fa.DHT = sa.DHT;
+      fa.DVNT = sa.DVNT;
+      fa.dh0 = dh0;
+      fa.N = N;
+      fa.units = (int)units;
+      fa.cu = cu_chunks;
+      fa.S = sa.S;
+      fa.H = H;
+      launch_bwd_scan<D>(st, NC, (const float*)sa.W, (const float*)sa.KgT, buf(B_DQG), buf(B_DKG),
+                         fa);
+    }
+  }
+  if (!frag)
+    hipLaunchKernelGGL((bwd_state<T, BT, D, BW, BP, BK>), dim3(units * (D / (16 * BW))),
+                       dim3(64 * (BW * BK + BP)), 0, st, sa);
   launch_mark(st);
   if (NC > 0) {
     // B3 (gdn2_bwd.py:126-210): one fused kernel with the D x D operands streamed
@@ -2284,8 +2313,32 @@ hipError_t launch_bwd(hipStream_t st, int B, int T_len, int H, const void* q, co
     // SIMD with 512 registers
     constexpr int BP = BK > 1 ? 4 : 2;
     const size_t units = cu_chunks ? (size_t)H * nseq : (size_t)B * H;
-    hipLaunchKernelGGL((bwd_state<T, BT, D, BW, BP, BK>), dim3(units * (D / (16 * BW))),
-                       dim3(64 * (BW * BK + BP)), 0, st, sa);
+    // B1: where the units leave CUs free, the scan over fragment tiles (the transposed
+    // tiles go into the DQG / DKG regions, which B3 writes afterwards); else bwd_state
+    bool frag = false;
+    if constexpr (sizeof(T) == 4) {
+      frag = !scan_rows(4, units, D);
+      if (frag) {
+        BScanArgs fa{};
+        fa.GL = sa.GL;
+        fa.DVPT = sa.DVPT;
+        fa.QDOT = sa.QDOT;
+        fa.dh_final = dh_final;
+        fa.DHT = sa.DHT;
+        fa.DVNT = sa.DVNT;
+        fa.dh0 = dh0;
+        fa.N = N;
+        fa.units = (int)units;
+        fa.cu = cu_chunks;
+        fa.S = sa.S;
+        fa.H = H;
+        launch_bwd_scan<D>(st, NC, (const float*)sa.W, (const float*)sa.KgT, buf(B_DQG), buf(B_DKG),
+                           fa);
+      }
+    }
+    if (!frag)
+      hipLaunchKernelGGL((bwd_state<T, BT, D, BW, BP, BK>), dim3(units * (D / (16 * BW))),
+                         dim3(64 * (BW * BK + BP)), 0, st, sa);
     launch_mark(st);
     if (NC > 0) {
       // B3, one fused kernel

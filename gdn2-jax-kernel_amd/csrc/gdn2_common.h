@@ -111,7 +111,7 @@ __device__ __forceinline__ Split8 split8(const f32x4& a, const f32x4& b) {
   }
   return s;
 }
-// Split pair layout of a float32 tile in LDS: in every 32-element run of a row
+// Split pair layout of a float32 tile: in every 32-element run of a row
 // (eight 16-byte chunks, chunk j = elements 4j .. 4j+3) the chunks j and 4 + j
 // (j < 4) are replaced by the hi and the lo parts of their eight elements, in
 // the order of split8(chunk j, chunk 4 + j).  A lane that reads chunks j and 4 + j
@@ -136,6 +136,36 @@ __device__ __forceinline__ Split4 split4(const f32x4& a) {
 #pragma unroll
   for (int e = 0; e < 4; ++e) s.lo[e] = (bf16_t)(a[e] - (float)s.hi[e]);
   return s;
+}
+// Operand-fragment order of a [R][K] tile that MFMA reads 16 rows x 32 k positions
+// at a time: fragment (rt, kk) is 64 lanes of 16 bytes, lane 16 lg + li holding row
+// 16 rt + li at the k positions {4 lg + r} and {16 + 4 lg + r} (the chained order of
+// kpos below).  Element offset of (row, k) for bfloat16 tiles:
+template <int K>
+__host__ __device__ constexpr int frag_off(int row, int k) {
+  return (((row / 16) * (K / 32) + k / 32) * 64 + ((k % 16) / 4) * 16 + row % 16) * 8 +
+         ((k / 16) % 2) * 4 + k % 4;
+}
+// Split float32 tiles hold each fragment's hi parts and then its lo parts (512
+// bfloat16 further): bfloat16 offset of the hi part of (row, k).
+template <int K>
+__host__ __device__ constexpr int split_frag_off(int row, int k) {
+  return frag_off<K>(row, k) + ((row / 16) * (K / 32) + k / 32) * 512;
+}
+// Elements k .. k + 3 (k a multiple of 4) of a row of a split tile in fragment order.
+template <int K>
+__device__ __forceinline__ void frag_store4(float* tile, int row, int k, const f32x4& v) {
+  const Split4 s = split4(v);
+  bf16_t* p = reinterpret_cast<bf16_t*>(tile) + split_frag_off<K>(row, k);
+  *reinterpret_cast<bf16x4*>(p) = s.hi;
+  *reinterpret_cast<bf16x4*>(p + 512) = s.lo;
+}
+template <int K>
+__device__ __forceinline__ void frag_store1(float* tile, int row, int k, float v) {
+  bf16_t* p = reinterpret_cast<bf16_t*>(tile) + split_frag_off<K>(row, k);
+  const bf16_t hi = (bf16_t)v;
+  p[0] = hi;
+  p[512] = (bf16_t)(v - (float)hi);
 }
 // Four consecutive elements 4m .. 4m+3 (m = e / 4) of a row stored in the split
 // pair layout, `row` the row's first byte.

@@ -42,10 +42,10 @@ struct PrepArgs {
   int T_len, H, N;
   long long NC;   // number of chunks, B*H*N
   float scale;
-  T* W;     // [cid][BT][D]; kPrepFull: bfloat16 -W in fragment order (gdn2_scan.h),
-            // float32 W in the split pair layout
-  T* UT;
-  T* KgT;   // [cid][D][BT]; float32: in the split pair layout (kPrepFull)
+  T* W;     // [cid][BT][D]; kPrepFull: -W in fragment order (gdn2_common.h), or (`rows`)
+            // W in the split pair layout
+  T* UT;    // [cid][D][BT], kPrepFull in fragment order (float32: 16 tokens each)
+  T* KgT;   // [cid][D][BT], kPrepFull in fragment order
   T* Qg;
   T* Aqk;
   float* GL;
@@ -56,6 +56,7 @@ struct PrepArgs {
                       // ([N+1], B = 1); rows past cstart[c+1] are neutral padding
   int frag;           // Qg and Aqk in operand-fragment order (qg_frag / aqk_frag):
                       // for the scan's output waves, which then read 1 KB per load
+  int rows;           // float32 W, kg^T, u^T in rows (scan_rows) instead of fragments
   int* sat_clear;     // segmented scan: its saturation flag, cleared here (the first
                       // launch of the call)
   // Stage modes (PrepMode): Akk output of kPrepScores, the given A of kPrepWy,
@@ -217,8 +218,8 @@ __global__ void __launch_bounds__(64 * prep_waves(BT), prep_min_blocks(sizeof(T)
     fwd_prep(PrepArgs<T, TG, TI> a) {
   static_assert(MODE == kPrepFull || (sizeof(T) == 4 && BT == 64),
                 "the stage modes run float32 tiles at chunk 64");
-  // float32 tiles of the forward: W and kg^T in the split pair layout of the
-  // float32 scans (gdn2_common.h), whose MFMA operands they are
+  // float32 tiles of the forward: W and kg^T as hi and lo fragments (gdn2_common.h),
+  // the operands of the float32 scans
   constexpr bool SPF = sizeof(T) == 4 && MODE == kPrepFull;
   using Op = typename Tr<T>::Op;
   constexpr int KC = Tr<T>::KC, KS = Tr<T>::KS;
@@ -483,7 +484,8 @@ __global__ void __launch_bounds__(64 * prep_waves(BT), prep_min_blocks(sizeof(T)
           if constexpr (MODE != kPrepScores) sKbdT[(d0 + ch) * TT_LD + t] = from_f<T>(bk * egc);
           const float kgv = sanitize(kv * ekh * sF1[I * DP + ch]);
           if constexpr (SPF) {
-            split_store1(reinterpret_cast<char*>(kgT + (size_t)(d0 + ch) * BT), t, kgv);
+            if (a.rows) split_store1(reinterpret_cast<char*>(kgT + (size_t)(d0 + ch) * BT), t, kgv);
+            else frag_store1<BT>(kgT, d0 + ch, t, kgv);
           } else if constexpr (MODE == kPrepFull) {
             kgT[frag_off<BT>(d0 + ch, t)] = from_f<T>(kgv);
           }
@@ -839,8 +841,11 @@ __global__ void __launch_bounds__(64 * prep_waves(BT), prep_min_blocks(sizeof(T)
         }
       }
       if constexpr (SPF) {
-        split_store4(reinterpret_cast<char*>(Wc + (size_t)(I * 16 + li) * D), dg + 4 * lg,
-                     sanitize4(accw));
+        if (a.rows)
+          split_store4(reinterpret_cast<char*>(Wc + (size_t)(I * 16 + li) * D), dg + 4 * lg,
+                       sanitize4(accw));
+        else
+          frag_store4<D>(Wc, I * 16 + li, dg + 4 * lg, -sanitize4(accw));
       } else if constexpr (sizeof(T) == 4) {
         store4(Wc + (size_t)(I * 16 + li) * D + dg + 4 * lg, sanitize4(accw));
       } else {
@@ -850,812 +855,13 @@ __global__ void __launch_bounds__(64 * prep_waves(BT), prep_min_blocks(sizeof(T)
         T* uc = a.UT + (size_t)cid * BT * D;
 #pragma unroll
         for (int r = 0; r < 4; ++r) uc[(size_t)(I * 16 + 4 * lg + r) * D + dg + li] = sanitize(accu[r]);
-      } else if constexpr (sizeof(T) == 4) {
-        store4(Uc + (size_t)(dg + li) * BT + I * 16 + 4 * lg, sanitize4(accu));
+      } else if constexpr (sizeof(T) == 4) {   // rows, or 16-token fragments
+        store4(Uc + (a.rows ? (dg + li) * BT + I * 16 + 4 * lg : ((dg / 16) * NB + I) * 256 + lane * 4),
+               sanitize4(accu));
       } else {
         store4(Uc + frag_off<BT>(dg + li, I * 16 + 4 * lg), sanitize4(accu));
       }
     }
-  }
-}
-
-// ---------------------------------------------------------------------------
-template <typename T>
-struct StateArgs {
-  const T* W;
-  const T* UT;
-  const T* KgT;
-  const float* GL;
-  const float* h0;  // nullable, (B,H,D,D)
-  int N;            // chunks per (b,h)
-  int S, L;         // segments per (b,h), chunks per segment (the last may be shorter)
-  int summary;      // segment-summary pass (S > 1): writes `seg`, no h^T / v_new^T
-  const float* hin; // S > 1 and !summary: segment entry states [bh][S][D][D]
-  float* seg;       // summary: [bh][S][2][D][D] = (end state, transition M_seg)
-  T* HT;
-  T* VnT;
-  float* h_final;
-  const int* cu;    // variable-length batch (B = 1): unit (h, sequence s) scans chunks
-                    // [cu[s], cu[s+1]); h0 / h_final are [s][h][D][D]
-  int H;
-  // Output waves (NO > 0): o = scale qg h_c + Aqk v_new formed in this kernel
-  // (h^T / v_new^T are then not written)
-  const T* Qg;
-  const T* Aqk;
-  float* out;
-  float scale;
-  int T_len;
-  const int* cstart;  // variable-length chunk table (see PrepArgs)
-  // Segmented scan (S > 1): `sat` is set to 1 when a clip of the carried state
-  // binds in a segmented pass (the segments' affine combination is exact only
-  // while none does); a pass with `gate` runs only if *gate is nonzero -- the
-  // serial scan that then replaces the segmented result
-  int* sat;
-  const int* gate;
-};
-
-// One workgroup = one (b,h) and 16*NW value columns: NW compute waves (16
-// columns each) and NP producer waves.  While the compute waves work on chunk
-// c, the producers stream chunk c+1 (W, kg^T, g_last and this workgroup's u^T
-// rows) into LDS with global_load_lds_dwordx4, wait for it and replace g_last
-// by e^{g_last}.  A wave
-// that issues that much memory traffic stalls at issue (at most 63 vector
-// memory instructions in flight per wave), so the compute waves issue none and
-// the traffic is split over several producers.  Two barriers per chunk: A
-// (chunk c resident, chunk c-1's buffers free) and B (u^T of chunk c copied to
-// registers, its buffer free).
-//
-// Segments (long sequences with few (b,h) pairs).  The chunk map
-// h -> M_c h + kg_c^T u_c, M_c = Diag(e^{g_last}) - kg_c^T W_c, is affine.  With
-// S > 1 segments of L chunks the scan runs in three launches: a summary pass
-// over all segments in parallel gives each segment's end state from h = 0 (h0
-// for segment 0) and, in NVS extra column slices that run the same recurrence
-// from the identity with u = 0 and no clipping, its transition M_seg; the
-// combine kernel chains the segment entry states; the final pass reruns every
-// segment from its entry state, writing h^T / v_new^T.  The combine is exact
-// while the +-1e4 clip of h does not bind; all three launches flag a binding
-// clip (StateArgs::sat), and a flagged call is finished by the serial scan.
-//
-// W / kg^T tiles are stored unpadded with the 16-byte chunks of row r
-// XOR-permuted by (r mod 16), so the 16 rows an MFMA operand read touches land
-// in distinct LDS banks.  Float32 tiles arrive in the split pair layout
-// (written so by fwd_prep, gdn2_common.h), and the two products run in the split
-// form: three bfloat16 MFMAs per 32-deep k step instead of eight float32 ones,
-// with h and v_new split once per chunk; the DMA moves the 16-byte chunks as
-// they are.  u^T is gathered straight into the order the compute
-// lanes read it (one contiguous 1 KB block per wave and row block).  The two
-// halves of the W / kg^T double buffer are separate __shared__ arrays selected
-// at compile time (the chunk loop is unrolled by two), so the compiler can see
-// that reads of one half never alias the DMA into the other.
-//
-// Where two buffers do not fit in LDS (float32 at D = 256: 128 KB per chunk)
-// the kernel runs single-buffered, with a third barrier E per chunk after the
-// compute waves' last reads.  The two tiles are read in different phases (W
-// before the K-split exchange X, kg^T after it), so the producers refill W and
-// u^T after X(c) and kg^T and g_last after E(c): each move hides behind the
-// other product, from L2 through the touch issued one chunk ahead.
-//
-// K-split (KS = 2): the two chained products of a chunk are the step's
-// critical path.  Each 16-column slice then has two compute waves, each
-// holding half of h's rows: both form their half of W h, exchange it through
-// LDS, form the same v_new = u - (W h)_lo - (W h)_hi and update their own rows
-// of h -- half the MFMA chain per wave, and all four SIMDs' matrix cores busy.
-// float32 exchanges through sX (barrier X, after B); bfloat16, whose two tile
-// buffers leave no room for sX, through the W tile of the current buffer once
-// every compute wave has read it (barriers X1, X2).  Not at D = 64 in
-// bfloat16, where the W tile is smaller than the exchanged partials.
-//
-// Output waves (NO > 0, inference: nothing reads h^T / v_new^T afterwards).
-// The outputs o = scale qg h_c + Aqk v_new of the workgroup's columns are
-// formed here instead of by fwd_out, so h_c and v_new never reach HBM.  The
-// compute waves keep h_c (bfloat16, natural d order) and v_new (chained order)
-// of chunk c in registers and put them into LDS (sHo, sVo) between barriers
-// A and B of chunk c+1; NO output waves, each owning the row blocks
-// {ow, NB-1-ow} (equal triangular work), read them from B(c+1) to A(c+2): one
-// row block while the compute waves form W h (B..X), the other during their h
-// update (after the last X barrier), so neither phase of the chain waits for
-// them.  q_g and Aqk rows come from global memory one chunk ahead, in the
-// operand-fragment order the prep writes for this path (qg_frag, aqk_frag).
-// Two barriers A(n), B(n) after the last chunk hand over its tiles.  Needs a
-// K-split (an X barrier per chunk) and both tile buffers.
-template <typename T, int BT, int D>
-constexpr int state_bufs() { return state_bufs_of(sizeof(T), BT, D); }
-template <typename T, int BT, int D>
-constexpr int state_ksplit() { return state_ksplit_of(sizeof(T), BT, D); }
-template <typename T, int BT, int D>
-constexpr int state_out_waves() { return state_out_waves_of(sizeof(T), BT, D); }
-
-template <typename T, int BT, int D, int NW, int NP, int KS, int NO = 0>
-__global__ void __launch_bounds__(64 * (NW * KS + NP + NO)) fwd_state(StateArgs<T> a) {
-  using Op = typename Tr<T>::Op;
-  constexpr int NB = BT / 16, NDT = D / 16;
-  constexpr int NVS = D / (16 * NW);
-  constexpr bool F32 = sizeof(T) == 4;
-  constexpr int WBYTES = BT * D * (int)sizeof(T);   // one tile (W or kg^T)
-  constexpr int BUF = 2 * WBYTES;                    // W + kg^T
-  constexpr int PIECES = BUF / 1024;                 // 1 KB DMA instructions per chunk
-  constexpr int NBUF = state_bufs<T, BT, D>();
-  constexpr int NCW = NW * KS;                       // compute waves
-  constexpr int NDH = NDT / KS;                      // row tiles of h per compute wave
-  static_assert(BUF % 1024 == 0, "tiles must split into 1 KB pieces");
-  // K-split exchange: through sX (float32, two parts; barrier X) or through the W
-  // tile of the current buffer (barriers X1, X2)
-  constexpr bool XSX = F32 && KS == 2;
-  constexpr int NXB = KS == 1 ? 0 : (XSX ? 1 : 2);
-  static_assert(KS == 1 || (NDT % KS == 0 && NB % KS == 0 &&
-                            (XSX || NCW * NB * 1024 <= WBYTES) &&
-                            (F32 || (KS == 2 && NDH % 2 == 0 && NB % 4 == 0))),
-                "K-split: the parts must split into whole k-steps, and the W tile "
-                "must hold the exchanged partials");
-  __shared__ __align__(16) char sbuf0[BUF];
-  __shared__ __align__(16) char sbuf1[NBUF == 2 ? BUF : 16];
-  // u^T in compute-lane order: 16 bytes per lane and row block (float32) or
-  // row-block pair (bfloat16, chained order)
-  constexpr int UB = F32 ? NB : NB / 2;              // u^T pieces per compute wave
-  __shared__ __align__(16) uint4 sU[NW * UB * 64];
-  __shared__ __align__(16) f32x4 sX[XSX ? NCW * NB * 64 : 1];   // K-split partials of W h
-  __shared__ __align__(16) float sGL0[D];
-  __shared__ __align__(16) float sGL1[NBUF == 2 ? D : 4];
-  __shared__ __align__(16) float sJunk[64];        // target of the L2 touches
-  // output waves: h_c^T [col][d] (natural order) and v_new^T [col][t] (chained
-  // order, as the v_new^T workspace tile) of the workgroup's columns
-  constexpr int PADO = 16 / (int)sizeof(T);
-  constexpr int HO_LD = D + PADO, VO_LD = BT + PADO;
-  __shared__ __align__(16) T sHo[NO > 0 ? 16 * NW * HO_LD : 8];
-  __shared__ __align__(16) T sVo[NO > 0 ? 16 * NW * VO_LD : 8];
-  static_assert(NO == 0 || (NXB > 0 && NBUF == 2 && NO == NB / 2),
-                "output waves need an X barrier per chunk, two tile buffers and NB/2 waves");
-
-  if (a.gate && *a.gate == 0) return;   // whole workgroups, before any barrier
-  const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lg = lane >> 4;
-  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // A unit is one (b,h) segment; it has NVS column slices (2 NVS in the summary
-  // pass, the second NVS carrying M).  Workgroups are dealt round-robin over the
-  // 8 XCDs (XCD = id mod 8): all slices of a unit go to one XCD so the W / kg^T
-  // tiles they all stream are fetched into that XCD's L2 once.
-  const int NSL = a.summary ? 2 * NVS : NVS;
-  int unit, vs;
-  bool one_xcd = false;   // all slices of the unit on this workgroup's XCD
-  {
-    const int nwg = gridDim.x, id = blockIdx.x;
-    const int per_xcd = nwg / 8;
-    if (nwg % 8 == 0 && per_xcd % NSL == 0) {
-      const int xcd = id % 8, slot = id / 8;
-      unit = xcd * (per_xcd / NSL) + slot / NSL;
-      vs = slot % NSL;
-      one_xcd = true;
-    } else {
-      unit = id / NSL;
-      vs = id % NSL;
-    }
-  }
-  const int bh = unit / a.S, sg = unit % a.S;
-  const bool mslice = vs >= NVS;             // summary pass: columns of M_seg
-  if (mslice && sg == 0) return;             // segment 0 starts from h0: no M needed
-  if (mslice) vs -= NVS;
-  int c0, n;                                 // chunks [c0, c0 + n) of this unit
-  if (a.cu) {
-    const SeqChunks sc = seq_chunks(a.cu, sg, a.N);
-    c0 = sc.c0;
-    n = sc.n;
-  } else {
-    c0 = sg * a.L;
-    n = a.N - c0;
-    n = n < a.L ? n : a.L;
-  }
-  n = n > 0 ? n : 0;
-
-  if constexpr (NO > 0) {
-    if (wv >= NCW + NP) {
-      // ---- output waves --------------------------------------------------------
-      // wave ow owns row blocks {ow, NB-1-ow} of every chunk and all 16 NW
-      // columns of the workgroup; out(c) is formed during chunk c+1 (after F for
-      // the last chunk) from sHo / sVo and the q_g / Aqk rows loaded one chunk
-      // ahead.  The barriers mirror the compute waves' A, B, X.. per chunk and F.
-      constexpr int TKC = Tr<T>::KC, TKS = Tr<T>::KS;
-      constexpr int OKD = D / TKS, OKT = BT / TKS;
-      const int ow = wv - NCW - NP;
-      const int hh = bh % a.H, bb = bh / a.H;
-      const size_t HD = (size_t)a.H * D;
-      auto oblock = [&](int i) { return i == 0 ? ow : NB - 1 - ow; };
-      Op qf[2][OKD], af[2][OKT];
-      // q_g and Aqk in operand-fragment order (the prep's frag layout): one
-      // 16-byte load per operand, 1 KB contiguous per wave
-      auto load_ops = [&](int c) __attribute__((always_inline)) {
-        const size_t cid = (size_t)bh * a.N + c0 + c;
-        const T* qc = a.Qg + cid * BT * D;
-        const T* ac = a.Aqk + cid * BT * BT;
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          const int It = oblock(i);
-#pragma unroll
-          for (int kg = 0; kg < OKD; ++kg) qf[i][kg] = op_load<T>(qc + qg_frag<T, BT, D>(It, kg, lane));
-          // Aqk blocks right of the diagonal block are never written: masked
-#pragma unroll
-          for (int kg = 0; kg < OKT; ++kg) {
-            if constexpr (sizeof(T) == 4) {
-              af[i][kg] = kg <= It ? op_load<T>(ac + aqk_frag<T, BT>(It, kg, lane)) : op_zero<T>();
-            } else {
-              af[i][kg] = 2 * kg <= It ? op_load<T>(ac + aqk_frag<T, BT>(It, 2 * kg, lane))
-                                       : op_zero<T>();
-            }
-          }
-        }
-      };
-      // out(c) rows of own row block i
-      auto emit = [&](int c, int i) __attribute__((always_inline)) {
-        const ChunkRows cr = chunk_rows(a.cstart, c0 + c, bb, a.T_len, BT);
-        float* obase = a.out + cr.row0 * HD + (size_t)hh * D + vs * 16 * NW;
-        {
-          const int It = oblock(i), t = It * 16 + li;
-          const int kgmax = (It * 16 + 15) / TKS;
-#pragma unroll
-          for (int vt = 0; vt < NW; ++vt) {
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int kg = 0; kg < OKD; ++kg)
-              mma(acc, op_load<T>(&sHo[(vt * 16 + li) * HO_LD + kg * TKS + lg * TKC]), qf[i][kg]);
-            acc *= a.scale;
-#pragma unroll
-            for (int kg = 0; kg < OKT; ++kg)
-              if (kg <= kgmax) {
-                Op y = af[i][kg];
-                if constexpr (sizeof(T) == 2) {
-                  if (2 * kg + 1 > It) {   // block 2kg+1 lies right of the diagonal
-#pragma unroll
-                    for (int e = 4; e < 8; ++e) y[e] = (T)0.f;
-                  }
-                }
-                mma(acc, op_load<T>(&sVo[(vt * 16 + li) * VO_LD + kg * TKS + lg * TKC]), y);
-              }
-            if (t < cr.valid) store4(obase + (size_t)t * HD + vt * 16 + 4 * lg, sanitize4(acc));
-          }
-        }
-      };
-      // chunk c-1's tiles are in sHo / sVo from B(c) to A(c+1): one row block
-      // while the compute waves form W h (B..X), the other during their h update
-      if (n > 0) load_ops(0);
-      for (int c = 0; c < n; ++c) {
-        lds_barrier();  // A(c)
-        lds_barrier();  // B(c)
-        if (c > 0) emit(c - 1, 0);
-        for (int x = 0; x < NXB; ++x) lds_barrier();  // X(c)
-        if (c > 0) {
-          emit(c - 1, 1);
-          load_ops(c);
-        }
-      }
-      lds_barrier();  // A(n)
-      lds_barrier();  // B(n)
-      if (n > 0) {
-        emit(n - 1, 0);
-        emit(n - 1, 1);
-      }
-      return;
-    }
-  }
-
-  if (wv >= NCW) {
-    // ---- producers ----------------------------------------------------------
-    // producer p moves W / kg^T pieces [p PP, (p+1) PP) and u^T blocks q = p mod NP
-    constexpr int ROWB_W = D * (int)sizeof(T), ROWB_K = BT * (int)sizeof(T);
-    constexpr int WPIECES = WBYTES / 1024;
-    constexpr int PP = PIECES / NP;
-    static_assert(PIECES % NP == 0 && (NW * UB) % NP == 0, "work must split evenly");
-    const int p = wv - NCW;
-    // parts: 1 the W / kg^T tiles and g_last, 2 the u^T blocks, 3 both
-    auto issue = [&](int c, char* base, float* gl, int parts = 3) __attribute__((always_inline)) {
-      const size_t cid = (size_t)bh * a.N + c0 + c;
-      const char* wsrc = reinterpret_cast<const char*>(a.W + cid * BT * D);
-      const char* ksrc = reinterpret_cast<const char*>(a.KgT + cid * D * BT);
-#pragma unroll
-      for (int i = 0; i < ((parts & 1) ? PP : 0); ++i) {
-        const int piece = p * PP + i;                      // wave-uniform
-        char* dst = base + piece * 1024;
-        if (piece < WPIECES) {
-          const int ib = piece * 1024 + lane * 16;
-          const int r = ib / ROWB_W, pch = (ib % ROWB_W) / 16;
-          constexpr int NCH = ROWB_W / 16, M = (NCH < 16 ? NCH : 16) - 1;
-          lds_dma16(wsrc + (size_t)r * ROWB_W + ((pch ^ (r & M)) * 16), dst);
-        } else {
-          const int ib = (piece - WPIECES) * 1024 + lane * 16;
-          const int r = ib / ROWB_K, pch = (ib % ROWB_K) / 16;
-          constexpr int NCH = ROWB_K / 16, M = (NCH < 16 ? NCH : 16) - 1;
-          lds_dma16(ksrc + (size_t)r * ROWB_K + ((pch ^ (r & M)) * 16), dst);
-        }
-      }
-      if ((parts & 1) && p == NP - 1 && lane < D / 4) lds_dma16(a.GL + cid * D + lane * 4, gl);
-      if (!(parts & 2)) return;
-      // u^T[col][t] for compute wave w, piece q: lane (li, lg) of that wave gets
-      // the 16 bytes at u^T[16 w + li][16 q + 4 lg] (float32: row block q) or
-      // [32 q + 8 lg] (bfloat16: row blocks 2q, 2q+1, chained), at sU[(w UB + q) 64 + lane]
-      if (mslice) return;  // M columns: u = 0
-      constexpr int EPP = 16 / sizeof(T);              // elements per piece per lane
-      const T* usrc = a.UT + cid * D * BT + (size_t)(vs * 16 * NW + li) * BT + EPP * lg;
-#pragma unroll
-      for (int j = 0; j < NW * UB / NP; ++j) {
-        const int q = j * NP + p, w = q / UB, it = q % UB;
-        lds_dma16(usrc + (size_t)w * 16 * BT + it * 4 * EPP, &sU[q * 64]);
-      }
-    };
-    // L2 touch of chunk c: one 4-byte DMA into a junk slot per 128-byte line of
-    // everything issue(c) will read, spread over the producers.  Issued one
-    // chunk ahead of the DMA, it turns the DMA's HBM latency into L2 latency.
-    // The W / kg^T lines are read by every column slice of the unit: when the
-    // slices share an XCD (one L2) slice v touches only the v-th share of them
-    // (a touch per line and workgroup cost the scan a fifth of its time), every
-    // slice its own u^T rows.
-    constexpr int LINE = 128;
-    constexpr int LW = WBYTES / LINE;                       // lines per W / kg^T tile
-    constexpr int LUR = BT * (int)sizeof(T) / LINE;         // lines per u^T row
-    constexpr int LU = 16 * NW * LUR;                       // this workgroup's u^T rows
-    constexpr int LG = (D * 4 + LINE - 1) / LINE;           // g_last
-    // At chunk 64 the output waves' q_g and Aqk tiles are touched too, shared
-    // among the slices like W / kg^T (the touch count assumes that sharing;
-    // without it, lines past the count are left to the loads themselves): a
-    // step there (about 1.7 us) is shorter than the HBM latency of the operand
-    // loads issued one step ahead (fused scan 0.265 -> 0.217 ms).  A chunk-128
-    // step lasts long enough, and the extra touches cost more than they save
-    // (0.205 -> 0.213 ms).
-    constexpr bool TQA = NO > 0 && BT == 64;
-    constexpr int LQ = TQA ? BT * D * (int)sizeof(T) / LINE : 0;    // q_g
-    constexpr int LA = TQA ? BT * BT * (int)sizeof(T) / LINE : 0;   // Aqk
-    constexpr int LSH = 2 * LW + LQ + LA;                   // lines shared by the slices
-    constexpr int LTOT = TQA ? (LSH + NVS - 1) / NVS + LU + LG   // at most (one slice)
-                             : LSH + LU + LG;
-    constexpr int NTP = ((LTOT + 63) / 64 + NP - 1) / NP;   // touch instructions per producer
-    const int vsl = vs + (mslice ? NVS : 0);                // slice index within the unit
-    const int lws = one_xcd ? (LSH + NSL - 1) / NSL : LSH;  // shared lines touched here
-    const int lw0 = one_xcd ? vsl * lws : 0;
-    const int ltot = lws + LU + LG;
-    auto touch = [&](int c) __attribute__((always_inline)) {
-      const size_t cid = (size_t)bh * a.N + c0 + c;
-      const char* wsrc = reinterpret_cast<const char*>(a.W + cid * BT * D);
-      const char* ksrc = reinterpret_cast<const char*>(a.KgT + cid * D * BT);
-      const char* qsrc = reinterpret_cast<const char*>(a.Qg + cid * BT * D);
-      const char* asrc = reinterpret_cast<const char*>(a.Aqk + cid * BT * BT);
-      const char* usrc =
-          reinterpret_cast<const char*>(a.UT + cid * D * BT + (size_t)vs * 16 * NW * BT);
-      const char* gsrc = reinterpret_cast<const char*>(a.GL + cid * D);
-#pragma unroll
-      for (int j = 0; j < NTP; ++j) {
-        int l = (j * NP + p) * 64 + lane;
-        l = l < ltot ? l : ltot - 1;
-        const int lw = min(lw0 + l, LSH - 1);                   // shared line
-        const char* sh = lw < LW ? wsrc + lw * LINE
-                       : lw < 2 * LW ? ksrc + (lw - LW) * LINE
-                       : lw < 2 * LW + LQ ? qsrc + (lw - 2 * LW) * LINE
-                       : asrc + (lw - 2 * LW - LQ) * LINE;
-        const char* src = l < lws ? sh
-                        : l < lws + LU ? usrc + (l - lws) * LINE
-                        : gsrc + (l - lws - LU) * LINE;
-        lds_dma4(src, sJunk);
-      }
-    };
-    // In flight at the top of chunk c: issue(c), then touch(c+1) if c+1 < n.
-    auto wait_chunk = [&](int c) __attribute__((always_inline)) {
-      if (c + 1 < n) wait_vmcnt<NTP>();
-      else wait_vmcnt<0>();
-    };
-    // The producers' data ordering is the explicit vmcnt wait; a plain barrier
-    // (no fence) keeps the compiler from also waiting for the L2 touches.
-    auto barrier = []() __attribute__((always_inline)) {
-      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    };
-    // g_last -> e^{g_last} in place, once per chunk, by the producer that moved it
-    auto exp_gl = [&](float* gl) __attribute__((always_inline)) {
-      if (p == NP - 1) {
-#pragma unroll
-        for (int i = 0; i < (D + 63) / 64; ++i)
-          if (i * 64 + lane < D) gl[i * 64 + lane] = __expf(gl[i * 64 + lane]);
-      }
-    };
-    if constexpr (NBUF == 1) {
-      // One tile buffer: W and u^T of chunk c+1 move in once barrier X(c) has
-      // passed (the compute waves are done with W(c) and u^T(c)), kg^T and g_last
-      // once E(c) has passed, so each move hides behind the other product of the
-      // chain (kg^T v_new of chunk c, then W h of chunk c+1).  Every producer
-      // moves the same counts: its share of the W pieces and u^T blocks, then its
-      // share of the kg^T pieces and of g_last, which it exponentiates itself.
-      constexpr int PPW = WPIECES / NP, PPK = (PIECES - WPIECES) / NP, GQ = D / NP;
-      static_assert(WPIECES % NP == 0 && (PIECES - WPIECES) % NP == 0 && NXB == 1 &&
-                        GQ % 4 == 0 && GQ <= 64,
-                    "single-buffer split: equal shares per producer, one X barrier");
-      auto piece_dma = [&](const char* wsrc, const char* ksrc, int piece) __attribute__((always_inline)) {
-        char* dst = sbuf0 + piece * 1024;
-        if (piece < WPIECES) {
-          const int ib = piece * 1024 + lane * 16;
-          const int r = ib / ROWB_W, pch = (ib % ROWB_W) / 16;
-          constexpr int NCH = ROWB_W / 16, M = (NCH < 16 ? NCH : 16) - 1;
-          lds_dma16(wsrc + (size_t)r * ROWB_W + ((pch ^ (r & M)) * 16), dst);
-        } else {
-          const int ib = (piece - WPIECES) * 1024 + lane * 16;
-          const int r = ib / ROWB_K, pch = (ib % ROWB_K) / 16;
-          constexpr int NCH = ROWB_K / 16, M = (NCH < 16 ? NCH : 16) - 1;
-          lds_dma16(ksrc + (size_t)r * ROWB_K + ((pch ^ (r & M)) * 16), dst);
-        }
-      };
-      auto issue_w = [&](int c) __attribute__((always_inline)) {
-        const size_t cid = (size_t)bh * a.N + c0 + c;
-        const char* wsrc = reinterpret_cast<const char*>(a.W + cid * BT * D);
-#pragma unroll
-        for (int i = 0; i < PPW; ++i) piece_dma(wsrc, nullptr, p * PPW + i);
-        if (mslice) return;  // M columns: u = 0
-        constexpr int EPP = 16 / sizeof(T);
-        const T* usrc = a.UT + cid * D * BT + (size_t)(vs * 16 * NW + li) * BT + EPP * lg;
-#pragma unroll
-        for (int j = 0; j < NW * UB / NP; ++j) {
-          const int q = j * NP + p, w = q / UB, it = q % UB;
-          lds_dma16(usrc + (size_t)w * 16 * BT + it * 4 * EPP, &sU[q * 64]);
-        }
-      };
-      auto issue_k = [&](int c) __attribute__((always_inline)) {
-        const size_t cid = (size_t)bh * a.N + c0 + c;
-        const char* ksrc = reinterpret_cast<const char*>(a.KgT + cid * D * BT);
-#pragma unroll
-        for (int i = 0; i < PPK; ++i) piece_dma(nullptr, ksrc, WPIECES + p * PPK + i);
-        if (lane < GQ / 4) lds_dma16(a.GL + cid * D + p * GQ + lane * 4, sGL0 + p * GQ);
-      };
-      auto exp_q = [&]() __attribute__((always_inline)) {
-        if (lane < GQ) sGL0[p * GQ + lane] = __expf(sGL0[p * GQ + lane]);
-      };
-      if (n > 0) {
-        issue_w(0);
-        issue_k(0);
-      }
-      if (n > 1) touch(1);
-      for (int c = 0; c < n; ++c) {
-        // in flight here (c > 0): W / u^T of chunk c, then kg^T / g_last of chunk
-        // c (PPK + 1), then touch(c+1) if c+1 < n (NTP)
-        const bool tch = c + 1 < n;
-        if (c == 0) {
-          if (tch) wait_vmcnt<NTP>();
-          else wait_vmcnt<0>();
-          exp_q();
-        } else {
-          if (tch) wait_vmcnt<PPK + 1 + NTP>();
-          else wait_vmcnt<PPK + 1>();
-        }
-        barrier();  // A(c): W(c), u^T(c) resident
-        barrier();  // B(c)
-        if (c > 0) {
-          if (tch) wait_vmcnt<NTP>();
-          else wait_vmcnt<0>();
-          exp_q();
-        }
-        barrier();  // X(c): kg^T(c), e^{g_last(c)} resident; W(c) no longer read
-        if (c + 1 < n) issue_w(c + 1);
-        barrier();  // E(c): kg^T(c) no longer read
-        if (c + 1 < n) {
-          issue_k(c + 1);
-          if (c + 2 < n) touch(c + 2);
-        }
-      }
-      return;
-    }
-    if (n > 0) issue(0, sbuf0, sGL0);
-    if (n > 1) touch(1);
-    // float32: the next chunk's W / kg^T / g_last move once A(c) has passed (their
-    // buffer was last read in chunk c-1), its u^T once B(c) has (one u^T buffer,
-    // read between A(c) and B(c)); the touch comes last, so waiting for all but
-    // the touch waits for both.  The MFMA-bound float32 step gains the head start
-    // (training scan 0.458 -> 0.437 ms); the latency-bound bfloat16 steps lost
-    // (0.210 -> 0.229 ms at chunk 128) and issue everything after B(c).
-    constexpr int EARLY = F32 ? 1 : 0;
-    for (int c = 0; c < n; c += 2) {
-      wait_chunk(c);
-      exp_gl(sGL0);
-      barrier();  // A(c)
-      if (EARLY && c + 1 < n) issue(c + 1, sbuf1, sGL1, 1);
-      barrier();  // B(c)
-      if (c + 1 < n) {
-        issue(c + 1, sbuf1, sGL1, EARLY ? 2 : 3);
-        if (c + 2 < n) touch(c + 2);
-        for (int x = 0; x < NXB; ++x) barrier();  // X(c)
-        wait_chunk(c + 1);
-        exp_gl(sGL1);
-        barrier();  // A(c+1)
-        if (EARLY && c + 2 < n) issue(c + 2, sbuf0, sGL0, 1);
-        barrier();  // B(c+1)
-        if (c + 2 < n) issue(c + 2, sbuf0, sGL0, EARLY ? 2 : 3);
-        if (c + 3 < n) touch(c + 3);
-        for (int x = 0; x < NXB; ++x) barrier();  // X(c+1)
-      } else {
-        for (int x = 0; x < NXB; ++x) barrier();  // X(c)
-      }
-    }
-    if constexpr (NO > 0) {
-      barrier();  // A(n)
-      barrier();  // B(n)
-    }
-    return;
-  }
-
-  // ---- compute waves ----------------------------------------------------------
-  const int wcol = wv % NW, ks = wv / NW;          // column slice, k-half (K-split)
-  const int col = vs * 16 * NW + wcol * 16 + li;
-  // element offset of logical (row r, element e) in a tile whose rows hold `re` elements
-  auto swz = [](int r, int e, int re) {
-    constexpr int EPC = 16 / sizeof(T);           // elements per 16-byte chunk
-    const int nchunk = re / EPC;
-    const int m = (nchunk < 16 ? nchunk : 16) - 1;
-    const int j = e / EPC;
-    return r * re + ((j ^ (r & m)) * EPC) + (e % EPC);
-  };
-
-  // entry state: h0 (or 0) for a plain pass and for segment 0 of the summary
-  // pass, 0 for later segments of the summary pass, the identity for M slices,
-  // the combined entry state in the final segmented pass
-  f32x4 h[NDH];   // row tiles at = ks NDH + i of this slice's h
-  const float* hsrc = a.cu ? (a.h0 ? a.h0 + ((size_t)sg * a.H + bh) * D * D : nullptr)
-                    : (a.S > 1 && !a.summary) ? a.hin + ((size_t)unit) * D * D
-                    : (sg == 0 && !mslice && a.h0) ? a.h0 + (size_t)bh * D * D : nullptr;
-  if (mslice) {
-#pragma unroll
-    for (int i = 0; i < NDH; ++i)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        h[i][r] = ((ks * NDH + i) * 16 + 4 * lg + r == col) ? 1.f : 0.f;
-  } else if (hsrc) {
-#pragma unroll
-    for (int i = 0; i < NDH; ++i)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        h[i][r] = sanitize(hsrc[(size_t)((ks * NDH + i) * 16 + 4 * lg + r) * D + col]);
-  } else {
-#pragma unroll
-    for (int i = 0; i < NDH; ++i) h[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
-  const bool write_tiles = !a.summary;
-  // segmented passes: whether a clip of the state bound (NaN included)
-  const bool track = a.sat != nullptr && !mslice;
-  bool bound = false;
-
-  // One chunk: v_new = u - W h, h <- e^{gl} h + kg^T v_new, with chunk c in `cur`.
-  // output waves: the pieces of chunk c-1's h^T / v_new^T this wave puts into
-  // sHo / sVo between barriers A(c) and B(c)
-  using HP = typename std::conditional<F32, f32x4, bf16x4>::type;
-  constexpr int NVP = F32 ? NB / KS : NB / 2 / KS;
-  HP hp[NO > 0 ? NDH : 1];
-  Op vp[NO > 0 ? NVP : 1];
-  auto put_tiles = [&]() __attribute__((always_inline)) {
-    const int lc = wcol * 16 + li;
-#pragma unroll
-    for (int i = 0; i < NDH; ++i)
-      *reinterpret_cast<HP*>(&sHo[lc * HO_LD + (ks * NDH + i) * 16 + 4 * lg]) = hp[i];
-#pragma unroll
-    for (int j = 0; j < NVP; ++j) {
-      if constexpr (F32) store4(&sVo[lc * VO_LD + (ks * NVP + j) * 16 + 4 * lg], vp[j]);
-      else *reinterpret_cast<Op*>(&sVo[lc * VO_LD + (ks * NVP + j) * 32 + 8 * lg]) = vp[j];
-    }
-  };
-
-  auto step = [&](int c, const char* cur, const float* eglc) __attribute__((always_inline)) {
-    const size_t cid = (size_t)bh * a.N + c0 + c;
-    __syncthreads();  // A(c)
-    f32x4 vn[NB];
-#pragma unroll
-    for (int q = 0; q < UB; ++q) {
-      const uint4 pc = sU[(wcol * UB + q) * 64 + lane];
-      if constexpr (F32) {
-        vn[q] = mslice ? f32x4{0.f, 0.f, 0.f, 0.f} : __builtin_bit_cast(f32x4, pc);
-      } else {
-        const bf16x8 e = __builtin_bit_cast(bf16x8, pc);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          vn[2 * q][r] = mslice ? 0.f : (float)e[r];
-          vn[2 * q + 1][r] = mslice ? 0.f : (float)e[4 + r];
-        }
-      }
-    }
-    if constexpr (NO > 0) {
-      if (c > 0) put_tiles();
-    }
-    __syncthreads();  // B(c)
-    const T* sW = reinterpret_cast<const T*>(cur);
-    const T* sK = reinterpret_cast<const T*>(cur + WBYTES);
-
-    T* hT = a.HT + cid * D * D + (size_t)col * D;
-    if (!write_tiles || NO > 0) {
-    } else if constexpr (F32) {
-#pragma unroll
-      for (int i = 0; i < NDH; ++i) store4(hT + (ks * NDH + i) * 16 + 4 * lg, h[i]);
-    } else {
-#pragma unroll
-      for (int p = 0; p < NDH / 2; ++p)
-        *reinterpret_cast<Op*>(hT + (ks * NDH / 2 + p) * 32 + 8 * lg) =
-            op_from_c(h[2 * p], h[2 * p + 1], (Op*)nullptr);
-    }
-
-    // v_new -= W h.  The NB row blocks are independent accumulators: the k-step
-    // loop is outermost, so consecutive MFMAs never wait on each other, and the
-    // next k-step's W operands are read while this one's MFMAs run.
-    {
-      constexpr int NKD = F32 ? NDH : NDH / 2;   // k-steps over this wave's d
-      Op hb[NKD];
-#pragma unroll
-      for (int kk = 0; kk < NKD; ++kk) {
-        if constexpr (F32) hb[kk] = h[kk];
-        else hb[kk] = op_from_c(h[2 * kk], h[2 * kk + 1], (Op*)nullptr);
-      }
-      auto wop = [&](int it, int kk) __attribute__((always_inline)) {
-        const int r = it * 16 + li;
-        if constexpr (F32) return load4f(&sW[swz(r, (ks * NDH + kk) * 16 + 4 * lg, D)]);
-        else return op_load<T>(&sW[swz(r, (ks * NKD + kk) * 32 + 8 * lg, D)]);
-      };
-      f32x4 acc[NB];
-      if constexpr (F32) {
-        // split form: h split once per chunk; the W tile holds the split pairs
-        // (chunks 2p, 2p+1 of a lane are one pair), all row blocks independent
-        static_assert(NKD % 2 == 0, "pairs of k-groups");
-        Split8 hs[NKD / 2];
-#pragma unroll
-        for (int p = 0; p < NKD / 2; ++p) hs[p] = split8(hb[2 * p], hb[2 * p + 1]);
-#pragma unroll
-        for (int it = 0; it < NB; ++it) acc[it] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int p = 0; p < NKD / 2; ++p)
-#pragma unroll
-          for (int it = 0; it < NB; ++it)
-            mma3(acc[it], split_read(wop(it, 2 * p), wop(it, 2 * p + 1)), hs[p]);
-      } else {
-        // bfloat16: one accumulator chain at a time (a chain of dependent
-        // 16x16x32 MFMAs issues faster than interleaved accumulators); the next
-        // row block's W operands are read while this one's chain runs
-        Op wc[NKD], wn[NKD];
-#pragma unroll
-        for (int kk = 0; kk < NKD; ++kk) wc[kk] = wop(0, kk);
-#pragma unroll
-        for (int it = 0; it < NB; ++it) {
-          if (it + 1 < NB) {
-#pragma unroll
-            for (int kk = 0; kk < NKD; ++kk) wn[kk] = wop(it + 1, kk);
-          }
-          acc[it] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int kk = 0; kk < NKD; ++kk) mma(acc[it], wc[kk], hb[kk]);
-#pragma unroll
-          for (int kk = 0; kk < NKD; ++kk) wc[kk] = wn[kk];
-        }
-      }
-      if constexpr (KS > 1) {
-        // exchange the parts; every wave of the slice sums them in the order of
-        // the k-parts, so all form the same v_new
-        f32x4* xb = sX;
-        if constexpr (!XSX) {
-          lds_barrier();  // X1(c): every compute wave is done with the W tile
-          xb = reinterpret_cast<f32x4*>(const_cast<char*>(cur));
-        }
-#pragma unroll
-        for (int it = 0; it < NB; ++it) xb[(wv * NB + it) * 64 + lane] = acc[it];
-        lds_barrier();  // X(c), X2(c)
-#pragma unroll
-        for (int it = 0; it < NB; ++it) {
-          f32x4 sum = ks == 0 ? acc[it] : xb[(wcol * NB + it) * 64 + lane];
-#pragma unroll
-          for (int q = 1; q < KS; ++q)
-            sum += ks == q ? acc[it] : xb[((q * NW + wcol) * NB + it) * 64 + lane];
-          vn[it] -= sum;
-        }
-      } else {
-#pragma unroll
-        for (int it = 0; it < NB; ++it) vn[it] -= acc[it];
-      }
-    }
-    T* vT = a.VnT + cid * D * BT + (size_t)col * BT;
-    if constexpr (NO > 0) {
-      // h_c and v_new of chunk c, kept for the output waves (put into LDS at the
-      // start of chunk c+1): h^T in natural d order (lane (li, lg) holds
-      // d = 16 i + 4 lg + r of row tile i), v_new^T in chained order
-#pragma unroll
-      for (int i = 0; i < NDH; ++i) {
-        if constexpr (F32) hp[i] = h[i];
-        else hp[i] = HP{(T)h[i][0], (T)h[i][1], (T)h[i][2], (T)h[i][3]};
-      }
-#pragma unroll
-      for (int j = 0; j < NVP; ++j) {
-        if constexpr (F32) vp[j] = vn[ks * NVP + j];
-        else vp[j] = op_from_c(vn[2 * (ks * NVP + j)], vn[2 * (ks * NVP + j) + 1], (Op*)nullptr);
-      }
-    } else if (!write_tiles) {
-    } else if constexpr (F32) {
-#pragma unroll
-      for (int it = ks * (NB / KS); it < (ks + 1) * (NB / KS); ++it)
-        store4(vT + it * 16 + 4 * lg, vn[it]);
-    } else {
-#pragma unroll
-      for (int p = ks * (NB / 2 / KS); p < (ks + 1) * (NB / 2 / KS); ++p)
-        *reinterpret_cast<Op*>(vT + p * 32 + 8 * lg) = op_from_c(vn[2 * p], vn[2 * p + 1], (Op*)nullptr);
-    }
-
-    // h <- e^{g_last} h + kg^T v_new (the row tiles of h are independent
-    // accumulators)
-    {
-      constexpr int NKT = F32 ? NB : NB / 2;     // k-steps over t
-#pragma unroll
-      for (int i = 0; i < NDH; ++i) {
-        const f32x4 egl = load4f(eglc + (ks * NDH + i) * 16 + 4 * lg);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) h[i][r] *= egl[r];
-      }
-      auto kop = [&](int i, int kk) __attribute__((always_inline)) {
-        const int r = (ks * NDH + i) * 16 + li;
-        if constexpr (F32) return load4f(&sK[swz(r, kk * 16 + 4 * lg, BT)]);
-        else return op_load<T>(&sK[swz(r, kk * 32 + 8 * lg, BT)]);
-      };
-      if constexpr (F32) {
-        // split form: v_new split once per chunk; the kg^T tile holds the split
-        // pairs, all row tiles of h independent
-        static_assert(NKT % 2 == 0, "pairs of k-groups");
-        Split8 vs2[NKT / 2];
-#pragma unroll
-        for (int p = 0; p < NKT / 2; ++p) vs2[p] = split8(vn[2 * p], vn[2 * p + 1]);
-#pragma unroll
-        for (int p = 0; p < NKT / 2; ++p)
-#pragma unroll
-          for (int at = 0; at < NDH; ++at)
-            mma3(h[at], split_read(kop(at, 2 * p), kop(at, 2 * p + 1)), vs2[p]);
-      } else {
-        // bfloat16: one chain per row tile of h, as for W h above
-        Op vb[NKT], kc2[NKT], kn2[NKT];
-#pragma unroll
-        for (int kk = 0; kk < NKT; ++kk) {
-          vb[kk] = op_from_c(vn[2 * kk], vn[2 * kk + 1], (Op*)nullptr);
-          kc2[kk] = kop(0, kk);
-        }
-#pragma unroll
-        for (int at = 0; at < NDH; ++at) {
-          if (at + 1 < NDH) {
-#pragma unroll
-            for (int kk = 0; kk < NKT; ++kk) kn2[kk] = kop(at + 1, kk);
-          }
-#pragma unroll
-          for (int kk = 0; kk < NKT; ++kk) mma(h[at], kc2[kk], vb[kk]);
-#pragma unroll
-          for (int kk = 0; kk < NKT; ++kk) kc2[kk] = kn2[kk];
-        }
-      }
-      if (!mslice) {
-        if (track) {
-#pragma unroll
-          for (int at = 0; at < NDH; ++at)
-#pragma unroll
-            for (int r2 = 0; r2 < 4; ++r2) bound = bound || !(fabsf(h[at][r2]) <= g_clip);
-        }
-#pragma unroll
-        for (int at = 0; at < NDH; ++at)
-#pragma unroll
-          for (int r2 = 0; r2 < 4; ++r2) h[at][r2] = sanitize(h[at][r2]);
-      }
-    }
-  };
-
-  if constexpr (NBUF == 1) {
-    for (int c = 0; c < n; ++c) {
-      step(c, sbuf0, sGL0);
-      __syncthreads();  // E(c)
-    }
-  } else {
-    for (int c = 0; c < n; c += 2) {
-      step(c, sbuf0, sGL0);
-      if (c + 1 < n) step(c + 1, sbuf1, sGL1);
-    }
-  }
-  if constexpr (NO > 0) {
-    __syncthreads();  // A(n): the output waves are done with chunk n-2's tiles
-    if (n > 0) put_tiles();
-    __syncthreads();  // B(n)
-  }
-  if (track && __ballot(bound) != 0 && lane == 0) *a.sat = 1;
-  float* hout = a.cu ? a.h_final + ((size_t)sg * a.H + bh) * D * D
-              : a.summary ? a.seg + ((size_t)unit * 2 + (mslice ? 1 : 0)) * D * D
-              : (sg == a.S - 1) ? a.h_final + (size_t)bh * D * D : nullptr;
-  if (hout) {
-#pragma unroll
-    for (int i = 0; i < NDH; ++i)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        hout[(size_t)((ks * NDH + i) * 16 + 4 * lg + r) * D + col] = h[i][r];
   }
 }
 
@@ -1873,25 +1079,68 @@ __global__ void __launch_bounds__(256) fwd_out(OutArgs<T> a) {
 // workgroup per CU (the shortest step: 0.8 us a chunk of 64 at D = 128, bfloat16,
 // against 1.1 with 32 columns), else of 32 (each loaded operand then feeds two
 // products: 48 (b,h) of 128 such chunks take 195 us against 280 with 16).
+// `rows`: float32 tiles laid out for fwd_state (scan_rows).
 template <typename T, int BT, int D>
-void launch_scan(hipStream_t st, ScanArgs<T> a, size_t units, bool outputs) {
+void launch_scan(hipStream_t st, ScanArgs<T> a, size_t units, bool outputs, bool rows,
+                 bool summary = false) {
   constexpr int KS = scan_ksplit(sizeof(T), D);
-  const int sm = a.summary ? 2 : 1;
+  const int sm = summary ? 2 : 1;
   a.units = (int)units;
   if (units == 0) return;
+  if constexpr (sizeof(T) == 4) {
+    if (rows) {
+      const dim3 grid((unsigned)(units * (D / 32) * sm));
+      if (summary)
+        hipLaunchKernelGGL((fwd_state<BT, D, true>), grid, dim3(512), 0, st, a);
+      else
+        hipLaunchKernelGGL((fwd_state<BT, D, false>), grid, dim3(512), 0, st, a);
+      return;
+    }
+  }
   auto go = [&](auto cpc) {
     constexpr int CPW = decltype(cpc)::value, NVS = D / (16 * CPW);
     constexpr int NO = scan_out_waves(sizeof(T), KS, CPW);
     const dim3 grid(scan_grid(units, NVS * sm));
-    if (outputs)
-      hipLaunchKernelGGL((fwd_scan<T, BT, D, KS, CPW, NO>), grid, dim3(64 * (KS + NO + 1)), 0,
-                         st, a);
+    if constexpr (scan_outputs(sizeof(T), D)) {
+      if (outputs) {
+        hipLaunchKernelGGL((fwd_scan<T, BT, D, KS, CPW, NO, false>), grid,
+                           dim3(64 * (KS + NO + 1)), 0, st, a);
+        return;
+      }
+    }
+    if (summary)
+      hipLaunchKernelGGL((fwd_scan<T, BT, D, KS, CPW, 0, true>), grid, dim3(64 * (KS + 1)), 0, st,
+                         a);
     else
-      hipLaunchKernelGGL((fwd_scan<T, BT, D, KS, CPW, 0>), grid, dim3(64 * (KS + 1)), 0, st, a);
+      hipLaunchKernelGGL((fwd_scan<T, BT, D, KS, CPW, 0, false>), grid, dim3(64 * (KS + 1)), 0,
+                         st, a);
   };
   if (units * sm * (D / 16) <= 256) go(std::integral_constant<int, 1>{});
   else go(std::integral_constant<int, 2>{});
 }
+
+// B1 on a forward's fragment tiles (the few units of scan_rows): the transposed
+// fragments into `kg` and `wt` ([cid][64][D] each), then the reverse scan.
+template <int D>
+hipError_t launch_bwd_scan(hipStream_t st, size_t nchunks, const float* W, const float* KgT,
+                           float* kg, float* wt, BScanArgs a) {
+  constexpr int BT = 64, KS = scan_ksplit(4, D);
+  if (nchunks > 0)
+    hipLaunchKernelGGL((frag_transpose<BT, D>), dim3((unsigned)(4 * nchunks)), dim3(256), 0, st,
+                       W, wt, KgT, kg, (int)nchunks);
+  a.Kg = kg;
+  a.WT = wt;
+  if (a.units > 0)
+    hipLaunchKernelGGL((bwd_scan<BT, D, KS>), dim3(scan_grid(a.units, D / 16)),
+                       dim3(64 * (KS + 1)), 0, st, a);
+  return hipGetLastError();
+}
+template hipError_t launch_bwd_scan<64>(hipStream_t, size_t, const float*, const float*, float*,
+                                        float*, BScanArgs);
+template hipError_t launch_bwd_scan<128>(hipStream_t, size_t, const float*, const float*, float*,
+                                         float*, BScanArgs);
+template hipError_t launch_bwd_scan<256>(hipStream_t, size_t, const float*, const float*, float*,
+                                         float*, BScanArgs);
 
 // ---------------------------------------------------------------------------
 // Host launchers (called from gdn2_api.cpp).
@@ -1904,7 +1153,6 @@ hipError_t launch_fwd(hipStream_t st, int B, int T_len, int H, const void* q, co
   const size_t NC = (size_t)B * H * N;
   // the segment count follows flags only (the workspace was sized from them): the
   // final pass of an inference forward is the 32-column scan with output waves
-  constexpr int NO = state_out_waves<T, BT, D>();
   const bool fuse_ws = scan_outputs(sizeof(T), D) && !(flags & 1);
   const int S_ws = vl ? 1
                       : state_segments((long long)B * H, N, D, (int)sizeof(T), (flags >> 8) & 0xff,
@@ -1914,6 +1162,7 @@ hipError_t launch_fwd(hipStream_t st, int B, int T_len, int H, const void* q, co
   // h^T / v_new^T tiles have no region (a variable-length workspace keeps them:
   // its size does not depend on flags)
   const bool fuse = fuse_ws && !a_dbg;
+  const bool rows = !fuse && scan_rows(sizeof(T), (size_t)B * H * (vl ? vl->nseq : 1), D);
   const size_t seg_units = S_ws > 1 ? (size_t)B * H * S_ws : 0;
   const FwdLayout L = fwd_layout(NC, BT, D, sizeof(T), seg_units, !(flags & kFwdNoARegion),
                                  !fuse || vl != nullptr);
@@ -1934,127 +1183,55 @@ hipError_t launch_fwd(hipStream_t st, int B, int T_len, int H, const void* q, co
                        (const TG*)g, T_len, H, N, (long long)NC, scale, W, UT, KgT, Qg, Aqk, GL,
                        a_dbg ? a_dbg : ((flags & 1) ? reinterpret_cast<float*>(ws + L.A)
                                                     : nullptr),
-                       (flags & 2) ? 1 : 0, vl ? vl->cstart : nullptr, fuse ? 1 : 0, sat};
+                       (flags & 2) ? 1 : 0, vl ? vl->cstart : nullptr, fuse ? 1 : 0, rows ? 1 : 0, sat};
     hipLaunchKernelGGL((fwd_prep<T, TG, BT, D, TI>), dim3(NC), dim3(64 * prep_waves(BT)), 0, st,
                        pa);
   }
   launch_mark(st);
-  if constexpr (sizeof(T) == 2) {
-    const size_t BH = (size_t)B * H;
-    ScanArgs<T> sa{};
-    sa.W = W;
-    sa.UT = UT;
-    sa.KgT = KgT;
-    sa.GL = GL;
-    sa.h0 = h0;
-    sa.N = N;
-    sa.S = 1;
-    sa.L = N;
-    sa.HT = HT;
-    sa.VnT = VnT;
-    sa.h_final = h_final;
-    sa.H = H;
-    sa.Qg = Qg;
-    sa.Aqk = Aqk;
-    sa.out = out;
-    sa.scale = scale;
-    sa.T_len = T_len;
-    if (vl) {   // one unit per (head, sequence)
-      sa.cu = vl->cu_chunks;
-      sa.cstart = vl->cstart;
-      sa.S = vl->nseq;
-      launch_scan<T, BT, D>(st, sa, BH * vl->nseq, fuse);
-    } else if (S_ws > 1) {
-      float* seg = reinterpret_cast<float*>(ws + L.SEG);            // [bh][S][2][D][D]
-      float* hin = seg + BH * S_ws * 2 * (size_t)D * D;              // [bh][S][D][D]
-      ScanArgs<T> pa = sa;
-      pa.S = S_ws;
-      pa.L = (N + S_ws - 1) / S_ws;
-      pa.sat = sat;
-      pa.summary = 1;
-      pa.seg = seg;
-      launch_scan<T, BT, D>(st, pa, BH * S_ws, false);
-      hipLaunchKernelGGL((seg_combine<D>), dim3(BH * (D / 16)), dim3(256), 0, st, seg, h0, hin,
-                         S_ws, sat);
-      pa.summary = 0;
-      pa.hin = hin;
-      launch_scan<T, BT, D>(st, pa, BH * S_ws, fuse);
-      // A clip of the state bound somewhere in the segmented passes: the segments'
-      // affine combination does not hold, and the serial scan recomputes everything
-      // the final pass wrote; otherwise its workgroups return at once
-      sa.gate = sat;
-      launch_scan<T, BT, D>(st, sa, BH, fuse);
-    } else {
-      launch_scan<T, BT, D>(st, sa, BH, fuse);
-    }
-  } else {
-  constexpr int SW = 2;  // compute waves (16 value columns each) per state workgroup
-  constexpr int SP = 4;  // producer waves (DMA issue: 4 beat 2 by 14 % on float32 scans)
-  constexpr int SK = state_ksplit<T, BT, D>();   // compute waves per column slice
-  constexpr int NVS = D / (16 * SW);
   const size_t BH = (size_t)B * H;
-  const int S = S_ws;
-  constexpr int NTH = 64 * (SW * SK + SP), NTHO = 64 * (SW * SK + SP + NO);
-  if (vl) {
-    // one unit per (head, sequence)
-    StateArgs<T> va{W,  UT,      KgT,     GL,     h0,           N,  vl->nseq, 0, 0, nullptr,
-                    nullptr, HT, VnT, h_final, vl->cu_chunks, H, Qg, Aqk, out, scale, T_len,
-                    vl->cstart};
-    if (vl->nseq > 0) {
-      if (fuse)
-        hipLaunchKernelGGL((fwd_state<T, BT, D, SW, SP, SK, NO>), dim3(BH * vl->nseq * NVS),
-                           dim3(NTHO), 0, st, va);
-      else
-        hipLaunchKernelGGL((fwd_state<T, BT, D, SW, SP, SK>), dim3(BH * vl->nseq * NVS),
-                           dim3(NTH), 0, st, va);
-    }
-  } else if (S > 1) {
-    // Segmented passes (several workgroups per CU's worth of units): bfloat16 at
-    // D >= 128 takes 64 columns per workgroup (four compute waves, no K-split),
-    // so the summary pass, which doubles the units with the M slices, fits the
-    // device in one round (1.1x faster than 32-column workgroups in two rounds)
-    constexpr int GW = seg_pass_cols(sizeof(T), D) / 16;
-    constexpr int GK = GW == SW ? SK : 1;
-    constexpr int GVS = D / (16 * GW);
-    const int Lseg = (N + S - 1) / S;
-    float* seg = reinterpret_cast<float*>(ws + L.SEG);          // [bh][S][2][D][D]
-    float* hin = seg + BH * S * 2 * (size_t)D * D;               // [bh][S][D][D]
-    StateArgs<T> sum{W, UT, KgT, GL, h0, N, S, Lseg, 1, nullptr, seg, HT, VnT, h_final,
-                     nullptr, H, Qg, Aqk, out, scale, T_len, nullptr, sat, nullptr};
-    hipLaunchKernelGGL((fwd_state<T, BT, D, GW, SP, GK>), dim3(BH * S * 2 * GVS),
-                       dim3(64 * (GW * GK + SP)), 0, st, sum);
+  ScanArgs<T> sa{};
+  sa.W = W;
+  sa.UT = UT;
+  sa.KgT = KgT;
+  sa.GL = GL;
+  sa.h0 = h0;
+  sa.N = N;
+  sa.S = 1;
+  sa.L = N;
+  sa.HT = HT;
+  sa.VnT = VnT;
+  sa.h_final = h_final;
+  sa.H = H;
+  sa.Qg = Qg;
+  sa.Aqk = Aqk;
+  sa.out = out;
+  sa.scale = scale;
+  sa.T_len = T_len;
+  if (vl) {   // one unit per (head, sequence)
+    sa.cu = vl->cu_chunks;
+    sa.cstart = vl->cstart;
+    sa.S = vl->nseq;
+    launch_scan<T, BT, D>(st, sa, BH * vl->nseq, fuse, rows);
+  } else if (S_ws > 1) {
+    float* seg = reinterpret_cast<float*>(ws + L.SEG);            // [bh][S][2][D][D]
+    float* hin = seg + BH * S_ws * 2 * (size_t)D * D;              // [bh][S][D][D]
+    ScanArgs<T> pa = sa;
+    pa.S = S_ws;
+    pa.L = (N + S_ws - 1) / S_ws;
+    pa.sat = sat;
+    pa.seg = seg;
+    launch_scan<T, BT, D>(st, pa, BH * S_ws, false, rows, true);
     hipLaunchKernelGGL((seg_combine<D>), dim3(BH * (D / 16)), dim3(256), 0, st, seg, h0, hin,
-                       S, sat);
-    StateArgs<T> fin{W, UT, KgT, GL, h0, N, S, Lseg, 0, hin, nullptr, HT, VnT, h_final,
-                     nullptr, H, Qg, Aqk, out, scale, T_len, nullptr, sat, nullptr};
-    if (fuse)   // final pass with output waves: 32-column workgroups
-      hipLaunchKernelGGL((fwd_state<T, BT, D, SW, SP, SK, NO>), dim3(BH * S * NVS), dim3(NTHO),
-                         0, st, fin);
-    else
-      hipLaunchKernelGGL((fwd_state<T, BT, D, GW, SP, GK>), dim3(BH * S * GVS),
-                         dim3(64 * (GW * GK + SP)), 0, st, fin);
+                       S_ws, sat);
+    pa.hin = hin;
+    launch_scan<T, BT, D>(st, pa, BH * S_ws, fuse, rows);
     // A clip of the state bound somewhere in the segmented passes: the segments'
-    // affine combination does not hold, and the serial scan (the plain pass below)
-    // recomputes everything the final pass wrote; otherwise its workgroups return
-    // at once
-    StateArgs<T> ser{W, UT, KgT, GL, h0, N, 1, N, 0, nullptr, nullptr, HT, VnT, h_final,
-                     nullptr, H, Qg, Aqk, out, scale, T_len, nullptr, nullptr, sat};
-    if (fuse)
-      hipLaunchKernelGGL((fwd_state<T, BT, D, SW, SP, SK, NO>), dim3(BH * NVS), dim3(NTHO), 0,
-                         st, ser);
-    else
-      hipLaunchKernelGGL((fwd_state<T, BT, D, SW, SP, SK>), dim3(BH * NVS), dim3(NTH), 0, st,
-                         ser);
+    // affine combination does not hold, and the serial scan recomputes everything
+    // the final pass wrote; otherwise its workgroups return at once
+    sa.gate = sat;
+    launch_scan<T, BT, D>(st, sa, BH, fuse, rows);
   } else {
-    StateArgs<T> sa{W, UT, KgT, GL, h0, N, 1, N, 0, nullptr, nullptr, HT, VnT, h_final,
-                    nullptr, H, Qg, Aqk, out, scale, T_len, nullptr};
-    if (fuse)
-      hipLaunchKernelGGL((fwd_state<T, BT, D, SW, SP, SK, NO>), dim3(BH * NVS), dim3(NTHO), 0,
-                         st, sa);
-    else
-      hipLaunchKernelGGL((fwd_state<T, BT, D, SW, SP, SK>), dim3(BH * NVS), dim3(NTH), 0, st,
-                         sa);
-  }
+    launch_scan<T, BT, D>(st, sa, BH, fuse, rows);
   }
   launch_mark(st);
   if (NC > 0 && !fuse) {
@@ -2168,15 +1345,24 @@ hipError_t launch_stage_combine(hipStream_t st, int B, int N, int H, const float
   const int T_len = N * BT;
   transpose_all(st, u, UT, NC, BT, D);
   transpose_all(st, kg, KgT, NC, BT, D);
-  // the scan's float32 tiles in the split pair layout, as fwd_prep writes them
+  // fwd_state's tiles in the split pair layout, as fwd_prep writes them (`rows`)
   split_runs(st, KgT, KgT, NC * D * BT / 32);
   split_runs(st, w_pseudo, Wsp, NC * BT * D / 32);
-  constexpr int SW = 2, SP = 4, SK = state_ksplit<float, BT, D>();
-  constexpr int NVS = D / (16 * SW);
-  StateArgs<float> sa{Wsp, UT, KgT, gc_last, h0, N, 1, N, 0, nullptr, nullptr, HT, VnT,
-                      h_final, nullptr, H, qg, aqk, out, scale, T_len, nullptr};
-  hipLaunchKernelGGL((fwd_state<float, BT, D, SW, SP, SK>), dim3((size_t)B * H * NVS),
-                     dim3(64 * (SW * SK + SP)), 0, st, sa);
+  ScanArgs<float> sa{};
+  sa.W = Wsp;
+  sa.UT = UT;
+  sa.KgT = KgT;
+  sa.GL = gc_last;
+  sa.h0 = h0;
+  sa.N = N;
+  sa.S = 1;
+  sa.L = N;
+  sa.HT = HT;
+  sa.VnT = VnT;
+  sa.h_final = h_final;
+  sa.H = H;
+  sa.T_len = T_len;
+  launch_scan<float, BT, D>(st, sa, (size_t)B * H, false, true);
   if (NC > 0) {
     OutArgs<float> oa{qg, aqk, HT, VnT, T_len, H, N, scale, out, nullptr};
     hipLaunchKernelGGL((fwd_out<float, BT, D>), dim3(NC * (D / out_cols<float, D>())),

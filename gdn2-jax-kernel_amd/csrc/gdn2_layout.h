@@ -165,32 +165,6 @@ constexpr SeqChunks seq_chunks(const int* cu, int s, int N) {
 // Columns of a segmented-pass workgroup: 64 for bfloat16 tiles at D >= 128, else 32.
 constexpr int seg_pass_cols(int esize, int D) { return esize == 2 && D >= 128 ? 64 : 32; }
 
-// Shape of the forward state-scan variants (fwd_state in gdn2_fwd.hip), here so
-// that the host's workspace size follows the same choices.  Tile buffers: two
-// when W and kg^T of two chunks fit LDS.  K-split: two compute waves per
-// column slice for float32, and for bfloat16 where the W tile holds the
-// exchanged partials.
-constexpr int state_bufs_of(int esize, int BT, int D) {
-  return 4 * BT * D * esize <= 132 * 1024 ? 2 : 1;
-}
-constexpr int state_ksplit_of(int esize, int BT, int D) {
-  return esize == 4 ? 2 : (4 * (BT / 16) * 1024 <= BT * D * 2 ? 2 : 1);
-}
-// Output waves of the inference scan (32 value columns per workgroup), which
-// then forms the outputs itself, or 0 where a separate output pass runs: no
-// K-split (bfloat16 at D = 64), a single tile buffer, or more LDS than 160 KB
-// (float32 at D >= 128).  The LDS count mirrors fwd_state's arrays.
-constexpr int state_out_waves_of(int esize, int BT, int D) {
-  const int NW = 2, PADT = 16 / esize;
-  const int tiles = 2 * 2 * BT * D * esize;                          // W, kg^T x 2
-  const int ub = NW * (esize == 4 ? BT / 16 : BT / 32) * 1024;       // u^T gather
-  const int xs = esize == 4 ? 2 * NW * (BT / 16) * 1024 : 0;        // K-split partials
-  const int fo = 16 * NW * (D + BT + 2 * PADT) * esize;             // staged h, v_new
-  const int lds = tiles + ub + xs + fo + 2 * D * 4 + 256;
-  return (state_ksplit_of(esize, BT, D) == 2 && state_bufs_of(esize, BT, D) == 2 &&
-          lds <= 160 * 1024) ? BT / 32 : 0;
-}
-
 // The forward scan (fwd_scan in gdn2_scan.h): whether an inference scan forms the
 // outputs itself (then no h^T / v_new^T tiles exist), here so that the host's
 // workspace size follows the same choice; its state waves per column slice (what
@@ -201,6 +175,16 @@ constexpr int scan_ksplit(int esize, int D) {
 }
 constexpr int scan_out_waves(int esize, int ksplit, int cpw) {
   return esize == 4 ? 4 : (ksplit == 1 && cpw == 1 ? 2 : 1);
+}
+
+// Float32 tiles W, kg^T and u^T in rows (W and kg^T in the split pair layout), for
+// fwd_state and bwd_state, instead of fragments, for fwd_scan: where `units` (b,h)
+// pairs or (head, sequence)s have more than one 16-column slice per CU.  Follows
+// shapes only, so that the backward knows what the forward kept.  At D = 128 on
+// 48 (b,h) of 128 chunks fwd_state takes 300 us and fwd_scan 368; on 24 of 32 75
+// and 44; at D = 256 on 12 of 64 405 and 175.
+constexpr bool scan_rows(int esize, size_t units, int D) {
+  return esize == 4 && units * (D / 16) > 256;
 }
 
 // Segments of the forward state scan for BH (b,h) pairs of N chunks with

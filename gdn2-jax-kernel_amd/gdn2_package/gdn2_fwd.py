@@ -282,15 +282,17 @@ def _residual_views(p: _Prepared, ws: torch.Tensor):
     idx = torch.arange(BT, device=p.device)
     causal = (idx[:, None] >= idx[None, :])
     # bfloat16 HT, VnT keep their last dimension in chained order (gdn2_common.h
-    # kpos); W (stored negated), UT, KgT are in operand-fragment order
-    # (gdn2_scan.h): undo it
+    # kpos).  W (negated), UT and KgT are in operand-fragment order (float32 W and
+    # KgT as hi and lo fragments, UT in fragments of 16 tokens), except float32
+    # tiles where the units fill the device (scan_rows in gdn2_layout.h): rows, W
+    # and KgT in the split pair layout.  Undo all of it.
     chained = p.tile_dt == torch.bfloat16
     nat = lambda x, n: x[..., _kpos_index(n, x.device)] if chained else x
-    # float32 W and KgT are in the scans' split pair layout: decode them
-    tile = lambda x: _frag_decode(x) if chained else x
-    spl = _frag_decode if chained else _split_decode
+    rows = not chained and B * H * (D // 16) > 256
+    spl = _frag_decode if chained else _split_decode if rows else _split_frag_decode
+    tile = _frag_decode if chained else (lambda x: x) if rows else _frag16_decode
     return {
-        "w_pseudo": f(spl(views["W"].view(*shp, BT, D))) * (-1.0 if chained else 1.0),
+        "w_pseudo": f(spl(views["W"].view(*shp, BT, D))) * (1.0 if rows else -1.0),
         "u": f(tile(views["UT"].view(*shp, D, BT)).transpose(-1, -2)),
         "kg": f(spl(views["KgT"].view(*shp, D, BT)).transpose(-1, -2)),
         "qg": f(views["Qg"].view(*shp, BT, D)),
@@ -302,14 +304,34 @@ def _residual_views(p: _Prepared, ws: torch.Tensor):
 
 
 def _split_decode(x: torch.Tensor) -> torch.Tensor:
-    """Rows of a float32 tile stored in the split pair layout of the float32
-    scans (csrc/gdn2_common.h) as float32: each 128-byte run of 32 elements holds
-    the bfloat16 hi parts (bytes 0-63) and lo parts (64-127), chunk j of each
-    part the elements 4j..4j+3 and 16+4j..16+4j+3; the value is hi + lo."""
+    """Rows stored in the split pair layout (csrc/gdn2_common.h) as float32: each
+    128-byte run of 32 elements holds the bfloat16 hi parts (bytes 0-63) and lo
+    parts (64-127), chunk j of each part the elements 4j..4j+3 and 16+4j..16+4j+3;
+    the value is hi + lo."""
     *lead, L = x.shape
     parts = x.contiguous().view(torch.bfloat16).reshape(*lead, L // 32, 2, 4, 2, 4).float()
     val = parts[..., 0, :, :, :] + parts[..., 1, :, :, :]          # (.., runs, j, half, slot)
     return val.transpose(-3, -2).reshape(*lead, L)                  # element 16 half + 4 j + slot
+
+
+def _split_frag_decode(x: torch.Tensor) -> torch.Tensor:
+    """Float32 tiles (..., R, K) stored as split fragments (csrc/gdn2_common.h) in
+    natural order: a fragment is 16 rows in the split pair layout with the (part,
+    chunk) of a row 16 rows apart."""
+    *lead, R, K = x.shape
+    y = x.contiguous().view(*lead, R // 16, K // 32, 2, 4, 16, 4)   # rt, kk, part, lg, li, 16 B
+    n = len(lead)
+    rows = y.permute(*range(n), n, n + 4, n + 1, n + 2, n + 3, n + 5)   # rt, li, kk, part, lg
+    return _split_decode(rows.reshape(*lead, R, K))
+
+
+def _frag16_decode(x: torch.Tensor) -> torch.Tensor:
+    """Float32 tiles (..., R, K) in fragments of 16 rows x 16 k, lane 16 lg + li =
+    row li, elements k = 4 lg + r."""
+    *lead, R, K = x.shape
+    y = x.contiguous().view(*lead, R // 16, K // 16, 4, 16, 4)   # rt, kt, lg, li, r
+    n = len(lead)
+    return y.permute(*range(n), n, n + 3, n + 1, n + 2, n + 4).reshape(*lead, R, K)
 
 
 def _frag_decode(x: torch.Tensor) -> torch.Tensor:

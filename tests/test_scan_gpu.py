@@ -36,3 +36,40 @@ def test_scan_edges(dtype, D, BT, chunks, short, wide):
     tol = 2e-2 if dtype == torch.bfloat16 else 1e-4
     assert np.allclose(out.cpu().numpy(), ro, rtol=tol, atol=tol)
     assert np.allclose(hf.cpu().numpy(), rh, rtol=tol, atol=tol)
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("chunks,short", [(1, 0), (2, 9), (3, 0), (4, 0)])
+@pytest.mark.parametrize("full", [False, True])
+def test_training_scan_edges(D, chunks, short, full):
+    """Forward and reverse scan of the training path on both sides of the rule that
+    lays its float32 tiles out (more units than one 16-column slice per CU holds:
+    rows, else fragments): all gradients, dh0 and a cotangent on h_final included,
+    against the float64 recurrence's."""
+    import gdn2_package as gp
+    B, H = 1, 256 // (D // 16) + 1 if full else 3
+    T = chunks * 64 - short
+    xs = O.make_inputs(B, T, H, D, seed=chunks * 10 + D)
+    rng = np.random.default_rng(5)
+    h0 = (0.3 * rng.standard_normal((B, H, D, D))).astype(np.float32)
+    do = rng.standard_normal((B, T, H, D)).astype(np.float32)
+    dhf = (0.1 * rng.standard_normal((B, H, D, D))).astype(np.float32)
+    dev = torch.device("cuda")
+    xt = [torch.tensor(x, device=dev, requires_grad=True) for x in (*xs, h0)]
+    out, hf = gp.gdn2_pallas_forward_trainable(*xt[:6], D ** -0.5, xt[6])
+    got = torch.autograd.grad([out, hf], xt, [torch.tensor(do, device=dev),
+                                              torch.tensor(dhf, device=dev)])
+    # the same in float64 by autograd of the token recurrence
+    x64 = [x.detach().double().requires_grad_(True) for x in xt]
+    q, k, v, w, b, g, s = x64
+    o = []
+    for t in range(T):
+        s = torch.exp(g[:, t]).unsqueeze(-1) * s
+        d = w[:, t] * v[:, t] - ((b[:, t] * k[:, t]).unsqueeze(-1) * s).sum(-2)
+        s = s + k[:, t].unsqueeze(-1) * d.unsqueeze(-2)
+        o.append(D ** -0.5 * (q[:, t].unsqueeze(-1) * s).sum(-2))
+    ref = torch.autograd.grad([torch.stack(o, 1), s], x64, [torch.tensor(do, device=dev).double(),
+                                                           torch.tensor(dhf, device=dev).double()])
+    for name, a, r in zip("q k v w b g h0".split(), got, ref):
+        # 1e-4 as the other float32 gradient tests
+        assert torch.all((a.double() - r).abs() <= 1e-4 + 1e-4 * r.abs()), name
