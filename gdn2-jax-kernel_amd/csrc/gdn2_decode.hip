@@ -6,35 +6,52 @@
 // are sanitized like every chunk state and output, gdn2_fwd.py:355-356).  The
 // state layout is h0 / h_final's: S[b][h][dk][dv] (gdn2_fwd.py:342).
 //
-// One 256-thread workgroup per (b,h) and slice of 16 state columns (B H D / 16
-// workgroups: enough to spread one decode step over the chip): thread (column
-// quad c4, row group rg) keeps D / 64 state rows of four columns in registers,
+// One 256-thread workgroup per (b,h) and slice of CS state columns: thread (column
+// quad c4, row group rg) keeps D CS / 1024 state rows of four columns in registers,
 // read and written with 16-byte accesses.  Both column reductions (pred and o)
 // run over the rows, so the columns split freely; they are summed over the row
 // groups of a wave by lane shuffles, then over the four waves in LDS.  The state
 // is read and written once (memory-bound); h_out may alias h_in.
+//
+// CS: a row of a slice should fill whole 128-byte lines (32 columns), or two
+// workgroups -- on different XCDs -- fetch and write back each line.  With 16, 32
+// and 64 columns (bfloat16 tokens, D = 128, state updated in place, kernels back to
+// back): 32 x 6 (b,h) 11.7, 6.2 and 6.1 us, 128 x 6 28.9, 19.4 and 16.6, 512 x 6
+// 95.9, 64.1 and 61.2 us (403 MB: 4.2, 6.3 and 6.6 TB/s); 8 x 6 at D = 256 10.7,
+// 6.4 and 6.6 us; 2 at D = 64 3.45, 3.75 and 4.40 us.  So: 64 columns from 512 such
+// workgroups on (two per CU), 16 where 32 would leave fewer than 32 workgroups.
 #include "gdn2_common.h"
 
 namespace gdn2 {
 
-template <int D>
-constexpr int decode_cols() { return 16; }
-
-// Sum of x over the lanes of a wave that hold the same column quad (lane & 3).
+// Sum of x over the lanes of a wave that hold the same column quad (lane mod C4).
+template <int C4>
 __device__ __forceinline__ f32x4 rowgroup_sum(f32x4 x) {
 #pragma unroll
-  for (int m = 4; m < 64; m *= 2)
+  for (int m = C4; m < 64; m *= 2)
 #pragma unroll
     for (int c = 0; c < 4; ++c) x[c] += __shfl_xor(x[c], m);
   return x;
 }
 
-template <typename T, typename TG, int D>
+// Sum over a thread's rows: rows 2j, 2j+1 are accumulated in p[j], then the p[j] are
+// added pairwise, so that wider slices (more rows per thread) round no more than
+// narrow ones.
+template <int N>
+__device__ __forceinline__ f32x4 pair_sum(f32x4 (&p)[N]) {
+#pragma unroll
+  for (int m = 1; m < N; m *= 2)
+#pragma unroll
+    for (int j = 0; j + m < N; j += 2 * m) p[j] += p[j + m];
+  return p[0];
+}
+
+template <typename T, typename TG, int D, int CS>
 __global__ void __launch_bounds__(256) decode_step(const T* q, const T* k, const T* v,
                                                    const T* w, const T* b, const TG* g,
                                                    float scale, const float* h_in,
                                                    float* h_out, float* out) {
-  constexpr int CS = decode_cols<D>(), NSL = D / CS;
+  constexpr int NSL = D / CS;
   constexpr int C4 = CS / 4, RG = 256 / C4, RPT = D / RG;   // row groups, rows per thread
   static_assert(RPT >= 1 && D % RG == 0, "rows must split over the row groups");
   __shared__ float sQ[D], sK[D], sBK[D], sEG[D];
@@ -62,17 +79,20 @@ __global__ void __launch_bounds__(256) decode_step(const T* q, const T* k, const
     sEG[i] = __expf(to_f(g[vo + i]));
   }
   __syncthreads();
-  f32x4 pred = {0.f, 0.f, 0.f, 0.f};
+  constexpr int NP = (RPT + 1) / 2;
+  f32x4 part[NP];
+#pragma unroll
+  for (int j = 0; j < NP; ++j) part[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int i = 0; i < RPT; ++i) {
     const int d = rg * RPT + i;
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       s[i][c] = sanitize(s[i][c]) * sEG[d];
-      pred[c] += sBK[d] * s[i][c];
+      part[i / 2][c] += sBK[d] * s[i][c];
     }
   }
-  pred = rowgroup_sum(pred);
+  f32x4 pred = rowgroup_sum<C4>(pair_sum(part));
   if (lane < C4) sRed[wave][lane] = pred;
   __syncthreads();
   pred = sRed[0][c4] + sRed[1][c4] + sRed[2][c4] + sRed[3][c4];
@@ -80,7 +100,8 @@ __global__ void __launch_bounds__(256) decode_step(const T* q, const T* k, const
 #pragma unroll
   for (int c = 0; c < 4; ++c) delta[c] = wv4[c] - pred[c];
   __syncthreads();  // every thread has read sRed
-  f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int j = 0; j < NP; ++j) part[j] = f32x4{0.f, 0.f, 0.f, 0.f};
   float* dst = h_out + bh * D * D;
 #pragma unroll
   for (int i = 0; i < RPT; ++i) {
@@ -89,11 +110,11 @@ __global__ void __launch_bounds__(256) decode_step(const T* q, const T* k, const
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       nv[c] = sanitize(s[i][c] + sK[d] * delta[c]);
-      o[c] += sQ[d] * nv[c];
+      part[i / 2][c] += sQ[d] * nv[c];
     }
     store4(dst + (size_t)d * D + col, nv);
   }
-  o = rowgroup_sum(o);
+  const f32x4 o = rowgroup_sum<C4>(pair_sum(part));
   if (lane < C4) sRed[wave][lane] = o;
   __syncthreads();
   if (tid < C4) {
@@ -107,10 +128,16 @@ hipError_t launch_decode(hipStream_t st, int B, int H, const void* q, const void
                          const void* v, const void* w, const void* b, const void* g,
                          float scale, const float* h_in, float* h_out, float* out) {
   launch_mark(st);
-  hipLaunchKernelGGL((decode_step<T, TG, D>), dim3((size_t)B * H * (D / decode_cols<D>())),
-                     dim3(256), 0, st,
-                     (const T*)q, (const T*)k, (const T*)v, (const T*)w, (const T*)b,
-                     (const TG*)g, scale, h_in, h_out, out);
+  auto go = [&](auto csc) {
+    constexpr int CS = decltype(csc)::value;
+    hipLaunchKernelGGL((decode_step<T, TG, D, CS>), dim3((size_t)B * H * (D / CS)), dim3(256), 0,
+                       st, (const T*)q, (const T*)k, (const T*)v, (const T*)w, (const T*)b,
+                       (const TG*)g, scale, h_in, h_out, out);
+  };
+  const size_t BH = (size_t)B * H;
+  if (BH * (D / 64) >= 512) go(std::integral_constant<int, 64>{});
+  else if (BH * (D / 32) >= 32) go(std::integral_constant<int, 32>{});
+  else go(std::integral_constant<int, 16>{});
   launch_mark(st);
   return hipGetLastError();
 }

@@ -82,3 +82,19 @@ def test_inplace_state_and_3d_inputs(dev):
     out, s = gp.gdn2_decode_step(*xt, 0.2, state=st, inplace=True)
     assert s.data_ptr() == st.data_ptr() and out.shape == (B, H, D)
     assert torch.equal(out, ref_out) and torch.equal(st, ref_state)
+
+
+@pytest.mark.parametrize("B,H,D", [(1, 15, 64), (1, 16, 64), (3, 5, 64), (64, 8, 64), (73, 7, 64),
+                                   (1, 7, 128), (2, 4, 128), (51, 5, 128), (32, 8, 128),
+                                   (1, 3, 256), (1, 4, 256), (127, 1, 256), (16, 8, 256)])
+def test_column_slices_match_recurrence(dev, B, H, D):
+    """Every column-slice width (16, 32, 64: by the number of workgroups), on both
+    sides of its lines, against the recurrence from a state."""
+    import gdn2_package as gp
+    xs = O.make_inputs(B, 1, H, D, seed=B + H)
+    h0 = (0.3 * np.random.default_rng(2).standard_normal((B, H, D, D))).astype(np.float32)
+    xt = [torch.tensor(x, device=dev) for x in xs]
+    out, h = gp.gdn2_decode_step(*xt, D ** -0.5, state=torch.tensor(h0, device=dev))
+    ro, rh = O.recurrent_fwd(*xs, D ** -0.5, h0=h0)
+    # float32 sums over D terms of magnitude <= 1: D 2^-24 < 2e-5
+    assert np.abs(out.cpu().numpy() - ro).max() < 2e-5 and np.abs(h.cpu().numpy() - rh).max() < 2e-5
