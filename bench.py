@@ -85,11 +85,10 @@ def kernel_table(dtype_bytes, chunk):
 
 
 # Inference forwards whose state scan forms the outputs itself (no fwd_out
-# launch): bfloat16 at D = 128 (chunk 64 or 128) and D = 256 (chunk 64), float32
-# at D = 64 -- the scan variants whose LDS holds the staged h / v_new tiles
-# (state_out_waves_of in gdn2_layout.h).  Their third launch interval is empty.
+# launch): bfloat16, and float32 at D = 64 (scan_outputs in gdn2_layout.h).  Their
+# third launch interval is empty.
 def fused_out(dtype_bytes, d):
-    return (dtype_bytes == 2 and d >= 128) or (dtype_bytes == 4 and d == 64)
+    return dtype_bytes == 2 or d == 64
 
 
 def name_kernels(kms, fused):
@@ -361,8 +360,9 @@ def mfma_from(run_dir):
     for (_, name), d in sorted(per.items()):
         if "gdn2" not in name:
             continue
-        short = next((k for k in ("fwd_prep", "fwd_state", "fwd_out", "bwd_b2", "bwd_state",
-                                  "bwd_wy", "gram_bwd") if k in name), name)
+        short = next((k for k in ("fwd_prep", "fwd_scan", "fwd_state", "fwd_out", "bwd_b2",
+                                  "bwd_scan", "bwd_state", "bwd_wy", "gram_bwd") if k in name),
+                     name)
         dt = "bf16" if ("DF16b" in name or "__bf16" in name or "bool" in name) else "fp32"
         f32 = 512 * d.get("SQ_INSTS_VALU_MFMA_MOPS_F32", 0)
         b16 = 512 * d.get("SQ_INSTS_VALU_MFMA_MOPS_BF16", 0)
@@ -663,7 +663,7 @@ def cpu_baseline(min_seconds=10.0, bwd_tokens=1024, bwd_min_seconds=8.0):
 COPY_BYTES = 1 << 30           # calibration copy: reads and writes this many bytes
 # the headline's launches (its scan forms the outputs): name matched in the
 # kernel symbol -> row of kernel_table
-KERNELS = {"fwd_prep": "fwd_prep", "fwd_state": "fwd_state_out"}
+KERNELS = {"fwd_prep": "fwd_prep", "fwd_scan": "fwd_state_out"}
 
 
 def pmc_run(steps, chunk=CHUNK):

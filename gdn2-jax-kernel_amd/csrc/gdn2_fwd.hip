@@ -2,8 +2,9 @@
 //
 //   fwd_prep  (one workgroup per chunk)      reference kernels A, B, C
 //             gdn2_fwd.py:99-139, 174-243, 264-295
-//   fwd_state (one workgroup per (b,h,64 value columns), serial over chunks)
-//             the state half of kernel D, gdn2_fwd.py:347-358
+//   fwd_scan  (one workgroup per (b,h) and 16 or 32 value columns, serial over
+//             chunks; gdn2_scan.h) the state half of kernel D, gdn2_fwd.py:347-358;
+//             float32 residuals on a full device: fwd_state
 //   fwd_out   (one workgroup per chunk)      the output half of kernel D,
 //             gdn2_fwd.py:349-353
 //
@@ -76,7 +77,8 @@ enum PrepMode { kPrepFull = 0, kPrepScores = 1, kPrepSolve = 2, kPrepWy = 3 };
 // Operand-fragment order of a chunk's q_g [BT][D] tile: the 16-byte operand
 // run a lane (li, lg) feeds a 16 x 16 MFMA for row block I and k-group j
 // (channels j*KS + lg*KC + e, e < KC) sits at fragment (I, j), lane 16 lg + li,
-// so the 64 lanes' operands of one fragment are 1 KB contiguous.
+// so the 64 lanes' operands of one fragment are 1 KB contiguous (bfloat16 tiles:
+// frag_off).
 template <typename T, int BT, int D>
 __host__ __device__ constexpr size_t qg_frag(int I, int j, int lane) {
   return ((size_t)(I * (D / Tr<T>::KS) + j) * 64 + lane) * Tr<T>::KC;

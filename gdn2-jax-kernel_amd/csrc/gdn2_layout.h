@@ -1,7 +1,7 @@
 // Workspace layout shared by the host API and the kernels.
 //
 // Every per-chunk tensor is stored chunk-major: chunk id cid = (b*H + h)*N + c,
-// then the tile.  Tiles are laid out so that each consumer reads 16-byte rows:
+// then the tile.  Tiles are laid out so that each consumer reads 16-byte runs:
 //   W    [cid][BT][D]   T     w_pseudo = A (b k e^gc)        (gdn2_fwd.py:278-279)
 //   UT   [cid][D][BT]   T     u^T, u = A (w v)               (gdn2_fwd.py:280)
 //   KgT  [cid][D][BT]   T     kg^T, kg = k e^(gc_last - gc)  (gdn2_fwd.py:285)
@@ -12,16 +12,19 @@
 //   VnT  [cid][D][BT]   T     v_new^T                         (gdn2_fwd.py:350)
 //   A    [cid][BT][BT]  f32   (I + Akk)^{-1}, written only for the backward
 //                             (GDN2_FWD_SAVE_A)               (gdn2_fwd.py:246-260)
-// T is float for float32 inputs and bfloat16 for bfloat16 inputs.  For
-// bfloat16 the last dimension of W, UT, KgT, HT and VnT (the index the serial state
-// pass contracts over or produces) is stored in chunk order kpos<T>() of
-// gdn2_common.h: within each 32-column block, column 16*half + 4*lg + r sits at
-// position 8*lg + 4*half + r.  float32 tiles are in natural order.
+// T is float for float32 inputs and bfloat16 for bfloat16 inputs.  W (negated), UT
+// and KgT are in the operand-fragment order of gdn2_common.h, float32 W and KgT as
+// split fragments, float32 UT in fragments of 16 tokens; where scan_rows holds,
+// float32 tiles are rows instead, W (not negated) and KgT in the split pair layout.
+// Qg and Aqk are fragments too where the scan forms the outputs (qg_frag,
+// aqk_frag).  The last dimension of bfloat16 HT and VnT is in chained order
+// (kpos<T>() of gdn2_common.h); float32 HT and VnT are in natural order.
 //
 // Backward workspace (all f32, chunk-major, one region per name):
 //   DAQK [BT][BT] dAqk (causal)      DVPT [D][BT] (Aqk^T do)^T    QDOT [D][D] (scale qg^T do)^T
 //   DHT  [D][D]  dh_{c+1}^T           DVNT [D][BT] dv_new^T
 //   DQG, DKG, DKBD [BT][D]            DAKK [BT][BT]
+//   (DQG and DKG hold bwd_scan's transposed kg and -W^T fragments until B3)
 //   SDH  [D]      sum_e dh_{c+1}[d][e] h_c[d][e]
 #pragma once
 

@@ -6,7 +6,7 @@ Same argument order and meaning as gdn2_fwd.py:400 (q,k,v,w,b,g of shape
 (B,T,H,D); ``scale`` a Python float; optional float32 ``h0`` (B,H,D,D)).
 ``out`` (B,T,H,D) and ``h_final`` (B,H,D,D) are float32 (gdn2_fwd.py:163-165,342).
 Tensors are torch tensors on the ROCm device; the compute runs in the gfx950
-HIP library libgdn2_hip.so (kernels fwd_prep / fwd_state / fwd_out).  There
+HIP library libgdn2_hip.so (kernels fwd_prep / fwd_scan / fwd_state / fwd_out).  There
 is no CPU fallback: without the library every call raises.
 
 Chunk size.  ``BT`` below plays the role of gdn2_fwd.py:29 but is read at call
