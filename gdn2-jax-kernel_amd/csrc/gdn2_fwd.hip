@@ -43,10 +43,10 @@ struct PrepArgs {
   int T_len, H, N;
   long long NC;   // number of chunks, B*H*N
   float scale;
-  T* W;     // [cid][BT][D]; kPrepFull: -W in fragment order (gdn2_common.h), or (`rows`)
+  T* W;     // [cid][BT][D]; kPrepFull: -W in fragment order (gdn2_common.h), kPrepRows:
             // W in the split pair layout
   T* UT;    // [cid][D][BT], kPrepFull in fragment order (float32: 16 tokens each)
-  T* KgT;   // [cid][D][BT], kPrepFull in fragment order
+  T* KgT;   // [cid][D][BT], kPrepFull in fragment order, kPrepRows in the split pair layout
   T* Qg;
   T* Aqk;
   float* GL;
@@ -57,7 +57,6 @@ struct PrepArgs {
                       // ([N+1], B = 1); rows past cstart[c+1] are neutral padding
   int frag;           // Qg and Aqk in operand-fragment order (qg_frag / aqk_frag):
                       // for the scan's output waves, which then read 1 KB per load
-  int rows;           // float32 W, kg^T, u^T in rows (scan_rows) instead of fragments
   int* sat_clear;     // segmented scan: its saturation flag, cleared here (the first
                       // launch of the call)
   // Stage modes (PrepMode): Akk output of kPrepScores, the given A of kPrepWy,
@@ -67,12 +66,15 @@ struct PrepArgs {
 };
 
 // What one fwd_prep launch computes.  kPrepFull: the forward's per-chunk tiles
-// (kernels A-C fused).  The reference's stages one at a time, float32 tiles in
+// (kernels A-C fused).  kPrepRows: the same with float32 W, kg^T and u^T in rows
+// (scan_rows) instead of fragments.  A mode and not an argument: the test at every
+// stored element cost the kernel 2 to 10 % (4 x 64 tokens, 12 heads of D = 128 26.9
+// against 25.3 us; 8 x 1024, 6 heads of D = 256 173 against 161).  The reference's stages one at a time, float32 tiles in
 // the reference's (B,H,N,BT,.) layout: kPrepScores Aqk and Akk
 // (build_chunk_scores_pallas, gdn2_fwd.py:142-170); kPrepSolve A = (I + Akk)^{-1}
 // from a given Akk (wy_solve_pallas, :246-260); kPrepWy w_pseudo, u, kg, qg,
 // gc_last from a given A (recompute_wy_pallas, :298-330).
-enum PrepMode { kPrepFull = 0, kPrepScores = 1, kPrepSolve = 2, kPrepWy = 3 };
+enum PrepMode { kPrepFull = 0, kPrepScores = 1, kPrepSolve = 2, kPrepWy = 3, kPrepRows = 4 };
 
 // Operand-fragment order of a chunk's q_g [BT][D] tile: the 16-byte operand
 // run a lane (li, lg) feeds a 16 x 16 MFMA for row block I and k-group j
@@ -219,10 +221,11 @@ template <typename T, typename TG, int BT, int D, typename TI, int MODE = kPrepF
 __global__ void __launch_bounds__(64 * prep_waves(BT), prep_min_blocks(sizeof(T), BT, D))
     fwd_prep(PrepArgs<T, TG, TI> a) {
   static_assert(MODE == kPrepFull || (sizeof(T) == 4 && BT == 64),
-                "the stage modes run float32 tiles at chunk 64");
-  // float32 tiles of the forward: W and kg^T as hi and lo fragments (gdn2_common.h),
-  // the operands of the float32 scans
-  constexpr bool SPF = sizeof(T) == 4 && MODE == kPrepFull;
+                "the stage and row modes run float32 tiles at chunk 64");
+  // float32 tiles of the forward: W and kg^T in hi and lo parts, as fragments or rows
+  // (gdn2_common.h), the operands of the float32 scans
+  constexpr bool ROWS = MODE == kPrepRows;
+  constexpr bool SPF = sizeof(T) == 4 && (MODE == kPrepFull || ROWS);
   using Op = typename Tr<T>::Op;
   constexpr int KC = Tr<T>::KC, KS = Tr<T>::KS;
   constexpr int NB = BT / 16;             // 16-token row blocks
@@ -486,8 +489,10 @@ __global__ void __launch_bounds__(64 * prep_waves(BT), prep_min_blocks(sizeof(T)
           if constexpr (MODE != kPrepScores) sKbdT[(d0 + ch) * TT_LD + t] = from_f<T>(bk * egc);
           const float kgv = sanitize(kv * ekh * sF1[I * DP + ch]);
           if constexpr (SPF) {
-            if (a.rows) split_store1(reinterpret_cast<char*>(kgT + (size_t)(d0 + ch) * BT), t, kgv);
-            else frag_store1<BT>(kgT, d0 + ch, t, kgv);
+            if constexpr (ROWS)
+              split_store1(reinterpret_cast<char*>(kgT + (size_t)(d0 + ch) * BT), t, kgv);
+            else
+              frag_store1<BT>(kgT, d0 + ch, t, kgv);
           } else if constexpr (MODE == kPrepFull) {
             kgT[frag_off<BT>(d0 + ch, t)] = from_f<T>(kgv);
           }
@@ -843,7 +848,7 @@ __global__ void __launch_bounds__(64 * prep_waves(BT), prep_min_blocks(sizeof(T)
         }
       }
       if constexpr (SPF) {
-        if (a.rows)
+        if constexpr (ROWS)
           split_store4(reinterpret_cast<char*>(Wc + (size_t)(I * 16 + li) * D), dg + 4 * lg,
                        sanitize4(accw));
         else
@@ -858,7 +863,7 @@ __global__ void __launch_bounds__(64 * prep_waves(BT), prep_min_blocks(sizeof(T)
 #pragma unroll
         for (int r = 0; r < 4; ++r) uc[(size_t)(I * 16 + 4 * lg + r) * D + dg + li] = sanitize(accu[r]);
       } else if constexpr (sizeof(T) == 4) {   // rows, or 16-token fragments
-        store4(Uc + (a.rows ? (dg + li) * BT + I * 16 + 4 * lg : ((dg / 16) * NB + I) * 256 + lane * 4),
+        store4(Uc + (ROWS ? (dg + li) * BT + I * 16 + 4 * lg : ((dg / 16) * NB + I) * 256 + lane * 4),
                sanitize4(accu));
       } else {
         store4(Uc + frag_off<BT>(dg + li, I * 16 + 4 * lg), sanitize4(accu));
@@ -1185,9 +1190,17 @@ hipError_t launch_fwd(hipStream_t st, int B, int T_len, int H, const void* q, co
                        (const TG*)g, T_len, H, N, (long long)NC, scale, W, UT, KgT, Qg, Aqk, GL,
                        a_dbg ? a_dbg : ((flags & 1) ? reinterpret_cast<float*>(ws + L.A)
                                                     : nullptr),
-                       (flags & 2) ? 1 : 0, vl ? vl->cstart : nullptr, fuse ? 1 : 0, rows ? 1 : 0, sat};
-    hipLaunchKernelGGL((fwd_prep<T, TG, BT, D, TI>), dim3(NC), dim3(64 * prep_waves(BT)), 0, st,
-                       pa);
+                       (flags & 2) ? 1 : 0, vl ? vl->cstart : nullptr, fuse ? 1 : 0, sat};
+    auto prep = [&](auto mode) {
+      hipLaunchKernelGGL((fwd_prep<T, TG, BT, D, TI, decltype(mode)::value>), dim3(NC),
+                         dim3(64 * prep_waves(BT)), 0, st, pa);
+    };
+    if constexpr (sizeof(T) == 4) {
+      if (rows) prep(std::integral_constant<int, kPrepRows>{});
+      else prep(std::integral_constant<int, kPrepFull>{});
+    } else {
+      prep(std::integral_constant<int, kPrepFull>{});
+    }
   }
   launch_mark(st);
   const size_t BH = (size_t)B * H;
