@@ -1086,6 +1086,10 @@ __global__ void __launch_bounds__(256) fwd_out(OutArgs<T> a) {
 // workgroup per CU (the shortest step: 0.8 us a chunk of 64 at D = 128, bfloat16,
 // against 1.1 with 32 columns), else of 32 (each loaded operand then feeds two
 // products: 48 (b,h) of 128 such chunks take 195 us against 280 with 16).
+// Float32 with output waves (D = 64) stays at 16 columns beyond that, with one output
+// wave instead of four and two workgroups per CU: 32 columns and four output waves
+// need more registers than seven waves leave (97 spilled, in the chunk loop; the scan
+// of 8 x 4096 tokens of 12 heads 352 us, of 8 x 2048 of 32 380; now 204 and 223).
 // `rows`: float32 tiles laid out for fwd_state (scan_rows).
 template <typename T, int BT, int D>
 void launch_scan(hipStream_t st, ScanArgs<T> a, size_t units, bool outputs, bool rows,
@@ -1104,17 +1108,26 @@ void launch_scan(hipStream_t st, ScanArgs<T> a, size_t units, bool outputs, bool
       return;
     }
   }
+  const bool few = units * sm * (D / 16) <= 256;
+  if constexpr (scan_outputs(sizeof(T), D)) {
+    if (outputs) {
+      auto out = [&](auto cpc, auto noc) {
+        constexpr int CPW = decltype(cpc)::value, NO = decltype(noc)::value;
+        hipLaunchKernelGGL((fwd_scan<T, BT, D, KS, CPW, NO, false>),
+                           dim3(scan_grid(units, D / (16 * CPW))), dim3(64 * (KS + NO + 1)), 0, st,
+                           a);
+      };
+      constexpr int CW = sizeof(T) == 4 ? 1 : 2;   // columns / 16 of a full device
+      if (few) out(std::integral_constant<int, 1>{},
+                   std::integral_constant<int, scan_out_waves(sizeof(T), KS, true)>{});
+      else out(std::integral_constant<int, CW>{},
+               std::integral_constant<int, scan_out_waves(sizeof(T), KS, false)>{});
+      return;
+    }
+  }
   auto go = [&](auto cpc) {
     constexpr int CPW = decltype(cpc)::value, NVS = D / (16 * CPW);
-    constexpr int NO = scan_out_waves(sizeof(T), KS, CPW);
     const dim3 grid(scan_grid(units, NVS * sm));
-    if constexpr (scan_outputs(sizeof(T), D)) {
-      if (outputs) {
-        hipLaunchKernelGGL((fwd_scan<T, BT, D, KS, CPW, NO, false>), grid,
-                           dim3(64 * (KS + NO + 1)), 0, st, a);
-        return;
-      }
-    }
     if (summary)
       hipLaunchKernelGGL((fwd_scan<T, BT, D, KS, CPW, 0, true>), grid, dim3(64 * (KS + 1)), 0, st,
                          a);
@@ -1122,7 +1135,7 @@ void launch_scan(hipStream_t st, ScanArgs<T> a, size_t units, bool outputs, bool
       hipLaunchKernelGGL((fwd_scan<T, BT, D, KS, CPW, 0, false>), grid, dim3(64 * (KS + 1)), 0,
                          st, a);
   };
-  if (units * sm * (D / 16) <= 256) go(std::integral_constant<int, 1>{});
+  if (few) go(std::integral_constant<int, 1>{});
   else go(std::integral_constant<int, 2>{});
 }
 

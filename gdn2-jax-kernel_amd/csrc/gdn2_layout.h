@@ -171,13 +171,19 @@ constexpr int seg_pass_cols(int esize, int D) { return esize == 2 && D >= 128 ? 
 // The forward scan (fwd_scan in gdn2_scan.h): whether an inference scan forms the
 // outputs itself (then no h^T / v_new^T tiles exist), here so that the host's
 // workspace size follows the same choice; its state waves per column slice (what
-// keeps a wave's operands in its registers) and its output waves.
+// keeps a wave's operands in its registers) and its output waves (`few`: every
+// 16-column slice has a CU of its own).
 constexpr bool scan_outputs(int esize, int D) { return esize == 2 || D == 64; }
 constexpr int scan_ksplit(int esize, int D) {
   return esize == 2 ? (D > 128 ? 2 : 1) : (D >= 256 ? 4 : 2);
 }
-constexpr int scan_out_waves(int esize, int ksplit, int cpw) {
-  return esize == 4 ? 4 : (ksplit == 1 && cpw == 1 ? 2 : 1);
+constexpr int scan_out_waves(int esize, int ksplit, bool few) {
+  return !few ? 1 : esize == 4 ? 4 : (ksplit == 1 ? 2 : 1);
+}
+// Workgroups per CU that fwd_scan is built for: two of the four-wave float32 form
+// with one output wave (256 registers a wave), else what its registers leave.
+constexpr int scan_per_cu(int esize, int out_waves) {
+  return esize == 4 && out_waves == 1 ? 2 : 1;
 }
 
 // Float32 tiles W, kg^T and u^T in rows (W and kg^T in the split pair layout), for

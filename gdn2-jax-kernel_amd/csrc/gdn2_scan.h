@@ -98,15 +98,21 @@ struct ScanArgs {
 // summed in the same order by every wave.  float32 tiles hold hi and lo fragments
 // and the products run in the split form (gdn2_common.h).
 // One barrier X(c) per chunk paces the waves and hands tiles over:
-//   * the helper brings the lines of a later chunk into L2 (one 4-byte DMA per
-//     128-byte line, shared among the unit's column slices, which run on one XCD)
-//     and puts e^{g_last}(c) into LDS before X(c);
+//   * the helper brings the lines of a later chunk into L2 (TOUCH: one 4-byte DMA
+//     per 128-byte line, shared among the unit's column slices, which run on one
+//     XCD) and puts e^{g_last}(c) into LDS before X(c);
 //   * the output waves form out(c) = scale qg h_c + Aqk v_new between X(c+1) and
 //     X(c+2).  h_c is written to LDS before X(c) (three slots), v_new between X(c)
 //     and X(c+1) (two slots), both in operand form.
 template <typename T, int BT, int D, int KS, int CPW, int NO, bool SUM>
-__global__ void __launch_bounds__(64 * (KS + NO + 1)) fwd_scan(ScanArgs<T> a) {
+__global__ void __launch_bounds__(64 * (KS + NO + 1), scan_per_cu(sizeof(T), NO))
+    fwd_scan(ScanArgs<T> a) {
   constexpr bool F32 = sizeof(T) == 4;
+  // Lines of later chunks are brought into L2 ahead of the loads, except where two
+  // workgroups share a CU: each then covers the other's waits, and the touches only
+  // add traffic (float32 D = 64, 8 x 4096 tokens of 12 heads: 436 us a call without,
+  // 440, 442 and 446 two, three and four chunks ahead).
+  constexpr bool TOUCH = scan_per_cu(sizeof(T), NO) == 1;
   using Op = typename Tr<T>::Op;                  // operands of the output products
   constexpr int PL = F32 ? 2 : 1;                 // hi and lo fragments of a tile
   constexpr int NB = BT / 16, NDT = D / 16, NKT = BT / 32;
@@ -218,7 +224,7 @@ __global__ void __launch_bounds__(64 * (KS + NO + 1)) fwd_scan(ScanArgs<T> a) {
     auto hstep = [&](int c, float* g) __attribute__((always_inline)) {
       put_eg(c + 1, g);
       load_gl(c + 3, g);
-      touch(c + AHEAD);
+      if constexpr (TOUCH) touch(c + AHEAD);
       lds_barrier();  // X(c)
     };
     if (n > 0) {
@@ -226,7 +232,8 @@ __global__ void __launch_bounds__(64 * (KS + NO + 1)) fwd_scan(ScanArgs<T> a) {
       put_eg(0, g0);
       load_gl(1, g1);
       load_gl(2, g0);
-      for (int c = 1; c < AHEAD; ++c) touch(c);
+      if constexpr (TOUCH)
+        for (int c = 1; c < AHEAD; ++c) touch(c);
     }
     lds_barrier();    // E
     int c = 0;
