@@ -111,8 +111,9 @@ __global__ void __launch_bounds__(64 * (KS + NO + 1), scan_per_cu(sizeof(T), NO)
   // Lines of later chunks are brought into L2 ahead of the loads, except where two
   // workgroups share a CU: each then covers the other's waits, and the touches only
   // add traffic (float32 D = 64, 8 x 4096 tokens of 12 heads: 436 us a call without,
-  // 440, 442 and 446 two, three and four chunks ahead).
-  constexpr bool TOUCH = scan_per_cu(sizeof(T), NO) == 1;
+  // 440, 442 and 446 two, three and four chunks ahead; bfloat16 summary pass, 131072
+  // tokens of 8 heads: 307 against 324 us at chunk 128, 323 against 345 at chunk 64).
+  constexpr bool TOUCH = scan_per_cu(sizeof(T), NO) == 1 && !(SUM && KS == 1 && CPW == 2);
   using Op = typename Tr<T>::Op;                  // operands of the output products
   constexpr int PL = F32 ? 2 : 1;                 // hi and lo fragments of a tile
   constexpr int NB = BT / 16, NDT = D / 16, NKT = BT / 32;
@@ -175,7 +176,15 @@ __global__ void __launch_bounds__(64 * (KS + NO + 1), scan_per_cu(sizeof(T), NO)
     constexpr int JPF = Tr<T>::KS / 16, NVK = NB / JPF;     // blocks per k-group, k-groups
     constexpr int LA = NO > 0 ? JPF * (NVK * (NVK + 1) / 2) * FPG : 0;
     constexpr int LSH = 2 * LW + (NO > 0 ? LW + LA : 0);  // W, kg^T (, q_g, Aqk): all slices
-    constexpr int AHEAD = BT >= 128 ? 2 : 4;               // chunks
+    // Chunk 128 on a full device: one chunk ahead, W by slice 0 and kg^T by slice 1.
+    // The lines of more chunks, or of more tiles, push one another out of the XCD's 4 MB
+    // (final pass of 131072 tokens of 8 heads, all tiles shared by all slices: 487 us
+    // two chunks ahead, 451 one; W and kg^T only, by four slices 453, by one 457, so
+    // 421).  With few units nothing is pushed out (4096 tokens of 6 heads 78 us a call,
+    // so 82).
+    constexpr bool TWO = BT >= 128 && CPW == 2;
+    constexpr int AHEAD = TWO ? 1 : BT >= 128 ? 2 : 4;     // chunks
+    static_assert(!TWO || (LW % 64 == 0 && NVS >= 2), "a slice touches a whole tile");
     const int lws = (LSH + NSL - 1) / NSL;                 // shared lines touched here
     constexpr int LMAX = (LSH + NVS - 1) / NVS + LU;
     constexpr int NTP = (LMAX + 63) / 64;
@@ -192,6 +201,14 @@ __global__ void __launch_bounds__(64 * (KS + NO + 1), scan_per_cu(sizeof(T), NO)
       const size_t cid = chunk_id(c);
       const char* wsrc = reinterpret_cast<const char*>(a.W + cid * BT * D);
       const char* ksrc = reinterpret_cast<const char*>(a.KgT + cid * D * BT);
+      if constexpr (TWO) {
+        if (vsl < 2) {
+          const char* src = vsl == 0 ? wsrc : ksrc;
+#pragma unroll
+          for (int j = 0; j < LW / 64; ++j) lds_dma4(src + (j * 64 + lane) * LINE, sJunk);
+        }
+        return;
+      }
       const char* qsrc = reinterpret_cast<const char*>(a.Qg + cid * BT * D);
       const char* asrc = reinterpret_cast<const char*>(a.Aqk + cid * BT * BT);
       const char* usrc =
