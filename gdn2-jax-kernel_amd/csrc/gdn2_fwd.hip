@@ -1090,6 +1090,10 @@ __global__ void __launch_bounds__(256) fwd_out(OutArgs<T> a) {
 // wave instead of four and two workgroups per CU: 32 columns and four output waves
 // need more registers than seven waves leave (97 spilled, in the chunk loop; the scan
 // of 8 x 4096 tokens of 12 heads 352 us, of 8 x 2048 of 32 380; now 204 and 223).
+// Float32 at D = 256, whose segmented passes fill the device, stays at 16 columns for
+// the same reason (five waves, 115 spilled; summary and final pass of 32768 tokens of
+// 4 heads 566 and 605 us with 32 columns, 393 and 355 with 16, 447 and 298 in
+// fwd_state on rows).
 // `rows`: float32 tiles laid out for fwd_state (scan_rows).
 template <typename T, int BT, int D>
 void launch_scan(hipStream_t st, ScanArgs<T> a, size_t units, bool outputs, bool rows,
@@ -1135,8 +1139,9 @@ void launch_scan(hipStream_t st, ScanArgs<T> a, size_t units, bool outputs, bool
       hipLaunchKernelGGL((fwd_scan<T, BT, D, KS, CPW, 0, false>), grid, dim3(64 * (KS + 1)), 0,
                          st, a);
   };
+  constexpr int CW = sizeof(T) == 4 && D > 128 ? 1 : 2;
   if (few) go(std::integral_constant<int, 1>{});
-  else go(std::integral_constant<int, 2>{});
+  else go(std::integral_constant<int, CW>{});
 }
 
 // B1 on a forward's fragment tiles (the few units of scan_rows): the transposed

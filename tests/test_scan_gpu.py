@@ -73,3 +73,41 @@ def test_training_scan_edges(D, chunks, short, full):
     for name, a, r in zip("q k v w b g h0".split(), got, ref):
         # 1e-4 as the other float32 gradient tests
         assert torch.all((a.double() - r).abs() <= 1e-4 + 1e-4 * r.abs()), name
+
+
+@pytest.mark.parametrize("dtype,D,BT,H,S,save", [
+    # more than 256 16-column slices in the final pass, with and without kept residuals
+    (torch.float32, 64, 64, 9, 8, False), (torch.float32, 64, 64, 9, 8, True),
+    (torch.float32, 128, 64, 5, 7, False), (torch.float32, 256, 64, 2, 9, False),
+    (torch.float32, 256, 64, 2, 9, True),
+    (torch.bfloat16, 64, 64, 9, 8, False), (torch.bfloat16, 64, 128, 9, 8, True),
+    (torch.bfloat16, 128, 64, 5, 7, True), (torch.bfloat16, 128, 128, 5, 7, False),
+    (torch.bfloat16, 256, 64, 2, 9, False), (torch.bfloat16, 256, 64, 2, 9, True),
+    # in the summary pass only (twice the slices)
+    (torch.float32, 128, 64, 3, 7, False), (torch.bfloat16, 256, 64, 1, 9, False),
+    (torch.bfloat16, 128, 128, 3, 7, False),
+    # forced segments where the (b,h) pairs alone fill the device (float32: rows)
+    (torch.float32, 64, 64, 65, 2, True), (torch.float32, 128, 64, 33, 2, False),
+    (torch.float32, 256, 64, 17, 2, False), (torch.bfloat16, 128, 64, 33, 2, False)])
+def test_segments_of_a_full_device(dtype, D, BT, H, S, save):
+    """The segmented scan's three passes in the forms that a full device takes, from a
+    state and with a short last chunk, against the serial scan and the recurrence."""
+    from gdn2_package import _lib
+    from gdn2_package.gdn2_fwd import _Prepared, _run_forward
+    T = (2 * S - 1) * BT - 9          # segments of two chunks, the last of one
+    xs = O.make_inputs(1, T, H, D, seed=D + H)
+    h0 = (0.3 * np.random.default_rng(8).standard_normal((1, H, D, D))).astype(np.float32)
+    dev = torch.device("cuda")
+    xt = [torch.tensor(x, device=dev).to(dtype) for x in xs[:5]] + [torch.tensor(xs[5], device=dev)]
+    p = _Prepared(*xt, D ** -0.5, torch.tensor(h0, device=dev), BT)
+    keep = _lib.FWD_SAVE_A if save else 0
+    out, hf, _, _ = _run_forward(p, flags=_lib.FWD_SEGMENTS(S) | keep)
+    out_1, hf_1, _, _ = _run_forward(p, flags=_lib.FWD_SEGMENTS(1) | keep)
+    # as test_fwd_gpu.py's segments: the order of the boundary-state products
+    near = 1e-5 if dtype == torch.float32 else 2e-3
+    assert torch.allclose(out, out_1, rtol=near, atol=near)
+    assert torch.allclose(hf, hf_1, rtol=near, atol=near)
+    ro, rh = O.recurrent_fwd(*[x.double().cpu().numpy() for x in xt], D ** -0.5, h0=h0)
+    tol = 2e-2 if dtype == torch.bfloat16 else 1e-4
+    assert np.allclose(out.cpu().numpy(), ro, rtol=tol, atol=tol)
+    assert np.allclose(hf.cpu().numpy(), rh, rtol=tol, atol=tol)

@@ -54,10 +54,11 @@ def scratch(tmp_path_factory):
 
 
 # mangled template arguments: fwd_scan<T, BT, D, KS, CPW, NO, SUM>
-@pytest.mark.parametrize("kernels", [
-    r"fwd_scanIfLi64ELi64E",        # float32, D = 64: every form
+@pytest.mark.parametrize("kernels,limit", [
+    (r"fwd_scanIfLi64ELi64E", 0),       # float32, D = 64: every form
+    (r"fwd_scanIfLi64ELi256E", 64),     # float32, D = 256: a few addresses, spilled once
 ])
-def test_scans_without_scratch(scratch, kernels):
+def test_scans_without_scratch(scratch, kernels, limit):
     found = {k: v for k, v in scratch.items() if re.search(kernels, k)}
     assert found
-    assert not any(found.values()), found
+    assert max(found.values()) <= limit, found
