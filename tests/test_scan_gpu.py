@@ -111,3 +111,41 @@ def test_segments_of_a_full_device(dtype, D, BT, H, S, save):
     tol = 2e-2 if dtype == torch.bfloat16 else 1e-4
     assert np.allclose(out.cpu().numpy(), ro, rtol=tol, atol=tol)
     assert np.allclose(hf.cpu().numpy(), rh, rtol=tol, atol=tol)
+
+
+@pytest.mark.parametrize("D,H,seqs", [(64, 5, 12), (64, 5, 13), (128, 3, 10), (128, 3, 11),
+                                      (256, 1, 16), (256, 1, 17)])
+def test_packed_training_layouts(D, H, seqs):
+    """Packed training with (head, sequence) counts on both sides of the rule that lays
+    the float32 tiles out, which the forward and the backward apply separately: every
+    gradient, dh0 included, against the float64 recurrence's; empty, short and exact
+    sequences among them."""
+    import gdn2_package as gp
+    lens = [(0, 17, 64, 65, 1, 100, 33)[i % 7] for i in range(seqs)]
+    T, cu = sum(lens), np.concatenate([[0], np.cumsum(lens)]).tolist()
+    xs = O.make_inputs(1, T, H, D, seed=D + seqs)
+    rng = np.random.default_rng(4)
+    h0 = (0.3 * rng.standard_normal((seqs, H, D, D))).astype(np.float32)
+    do = rng.standard_normal((1, T, H, D)).astype(np.float32)
+    dhf = (0.1 * rng.standard_normal((seqs, H, D, D))).astype(np.float32)
+    dev = torch.device("cuda")
+    xt = [torch.tensor(x, device=dev, requires_grad=True) for x in (*xs, h0)]
+    dt, dht = torch.tensor(do, device=dev), torch.tensor(dhf, device=dev)
+    out, hf = gp.gdn2_pallas_forward_varlen_trainable(*xt[:6], D ** -0.5, cu, xt[6])
+    got = torch.autograd.grad([out, hf], xt, [dt, dht])
+    x64 = [x.detach().double().requires_grad_(True) for x in xt]
+    q, k, v, w, b, g, s0 = x64
+    o, ends = [], []
+    for i, (a, e) in enumerate(zip(cu, cu[1:])):
+        s = s0[i]
+        for t in range(a, e):
+            s = torch.exp(g[0, t]).unsqueeze(-1) * s
+            d = w[0, t] * v[0, t] - ((b[0, t] * k[0, t]).unsqueeze(-1) * s).sum(-2)
+            s = s + k[0, t].unsqueeze(-1) * d.unsqueeze(-2)
+            o.append(D ** -0.5 * (q[0, t].unsqueeze(-1) * s).sum(-2))
+        ends.append(s)
+    ref = torch.autograd.grad([torch.stack(o)[None], torch.stack(ends)], x64,
+                              [dt.double(), dht.double()])
+    for name, x, r in zip("q k v w b g h0".split(), got, ref):
+        # 1e-4 as the other float32 gradient tests
+        assert torch.all((x.double() - r).abs() <= 1e-4 + 1e-4 * r.abs()), name
