@@ -899,7 +899,7 @@ __global__ void __launch_bounds__(256) seg_combine(const float* seg, const float
     sHT[cc * (D + 4) + r] = e0;
   }
   __syncthreads();
-  bool bound = false;   // a clip of an entry state bound (see StateArgs::sat)
+  bool bound = false;   // a clip of an entry state bound (see ScanArgs::sat)
   // M and e of a step do not depend on the state: loaded one segment ahead
   constexpr int NJ = (NDT + 3) / 4;
   f32x4 mn[NJ][NDT], en[NJ];
@@ -1176,14 +1176,14 @@ hipError_t launch_fwd(hipStream_t st, int B, int T_len, int H, const void* q, co
                       float* a_dbg, int flags, const Varlen* vl) {
   const int N = vl ? vl->total_chunks : (T_len + BT - 1) / BT;
   const size_t NC = (size_t)B * H * N;
-  // the segment count follows flags only (the workspace was sized from them): the
-  // final pass of an inference forward is the 32-column scan with output waves
+  // the segment count follows shapes and flags only (the workspace was sized from them)
   const bool fuse_ws = scan_outputs(sizeof(T), D) && !(flags & 1);
   const int S_ws = vl ? 1
                       : state_segments((long long)B * H, N, D, (int)sizeof(T), (flags >> 8) & 0xff,
                                        fuse_ws ? 32 : seg_pass_cols(sizeof(T), D));
-  // Inference (no residuals kept): the scan forms the outputs itself where its
-  // variant has output waves (state_out_waves), fwd_out is not launched and the
+  const int S = scan_segments(S_ws, (long long)B * H, N, D, (int)sizeof(T), (flags >> 8) & 0xff);
+  // Inference (no residuals kept): the scan forms the outputs itself where it has
+  // output waves (scan_outputs), fwd_out is not launched and the
   // h^T / v_new^T tiles have no region (a variable-length workspace keeps them:
   // its size does not depend on flags)
   const bool fuse = fuse_ws && !a_dbg;
@@ -1245,19 +1245,19 @@ hipError_t launch_fwd(hipStream_t st, int B, int T_len, int H, const void* q, co
     sa.cstart = vl->cstart;
     sa.S = vl->nseq;
     launch_scan<T, BT, D>(st, sa, BH * vl->nseq, fuse, rows);
-  } else if (S_ws > 1) {
+  } else if (S > 1) {
     float* seg = reinterpret_cast<float*>(ws + L.SEG);            // [bh][S][2][D][D]
-    float* hin = seg + BH * S_ws * 2 * (size_t)D * D;              // [bh][S][D][D]
+    float* hin = seg + BH * S * 2 * (size_t)D * D;                 // [bh][S][D][D]
     ScanArgs<T> pa = sa;
-    pa.S = S_ws;
-    pa.L = (N + S_ws - 1) / S_ws;
+    pa.S = S;
+    pa.L = (N + S - 1) / S;
     pa.sat = sat;
     pa.seg = seg;
-    launch_scan<T, BT, D>(st, pa, BH * S_ws, false, rows, true);
+    launch_scan<T, BT, D>(st, pa, BH * S, false, rows, true);
     hipLaunchKernelGGL((seg_combine<D>), dim3(BH * (D / 16)), dim3(256), 0, st, seg, h0, hin,
-                       S_ws, sat);
+                       S, sat);
     pa.hin = hin;
-    launch_scan<T, BT, D>(st, pa, BH * S_ws, fuse, rows);
+    launch_scan<T, BT, D>(st, pa, BH * S, fuse, rows);
     // A clip of the state bound somewhere in the segmented passes: the segments'
     // affine combination does not hold, and the serial scan recomputes everything
     // the final pass wrote; otherwise its workgroups return at once

@@ -165,7 +165,9 @@ constexpr SeqChunks seq_chunks(const int* cu, int s, int N) {
   return SeqChunks{c0, n > 0 ? (int)n : 0};
 }
 
-// Columns of a segmented-pass workgroup: 64 for bfloat16 tiles at D >= 128, else 32.
+// Columns by which a residual-keeping call's SEG region is sized: 64 for bfloat16 tiles
+// at D >= 128, else 32.  The passes are 32 columns wide and run the segments that
+// width asks for (scan_segments), never more than the region has.
 constexpr int seg_pass_cols(int esize, int D) { return esize == 2 && D >= 128 ? 64 : 32; }
 
 // The forward scan (fwd_scan in gdn2_scan.h): whether an inference scan forms the
@@ -198,7 +200,7 @@ constexpr bool scan_rows(int esize, size_t units, int D) {
 
 // Segments of the forward state scan for BH (b,h) pairs of N chunks with
 // `esize`-byte tiles, whose final pass runs workgroups of `final_cols` value
-// columns (seg_pass_cols, or 32 for the inference scan with output waves).
+// columns.
 // Automatic choice: as many as fill a 256-CU device in the final pass (BH *
 // D/final_cols workgroups per segment), each at least 16 chunks, and only when
 // that gives 4 or more (the segmented scan costs about 3/S of the serial chain
@@ -220,6 +222,15 @@ inline int state_segments(long long BH, int N, int D, int esize, int forced, int
   if (s < 1) s = 1;
   const long long len = (N + s - 1) / s;
   return (int)((N + len - 1) / (len > 0 ? len : 1));
+}
+
+// Segments a call runs in a workspace sized for `ws_segments`: those of the 32-column
+// passes.  The finer split of a bfloat16 SEG region (seg_pass_cols) is slower: 131072
+// tokens of 8 heads at chunk 128 2000 us in 16 segments, 1970 in 8; 32768 of 4 heads of
+// D = 256 865 in 16, 724 in 8; 16384 of 12 heads of D = 256 1048 in 4, 848 in one.
+inline int scan_segments(int ws_segments, long long BH, int N, int D, int esize, int forced) {
+  const int s = state_segments(BH, N, D, esize, forced, 32);
+  return s < ws_segments ? s : ws_segments;
 }
 
 }  // namespace gdn2

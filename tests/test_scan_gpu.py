@@ -149,3 +149,20 @@ def test_packed_training_layouts(D, H, seqs):
     for name, x, r in zip("q k v w b g h0".split(), got, ref):
         # 1e-4 as the other float32 gradient tests
         assert torch.all((x.double() - r).abs() <= 1e-4 + 1e-4 * r.abs()), name
+
+
+@pytest.mark.parametrize("D,H,T,S", [(128, 8, 16384, 8), (256, 12, 4096, 1)])
+def test_segments_of_a_residual_keeping_call(D, H, T, S):
+    """A bfloat16 forward that keeps its residuals runs the segments that its 32-column
+    passes ask for, whatever its workspace is sized for: bit for bit the forced count."""
+    from gdn2_package import _lib
+    from gdn2_package.gdn2_fwd import _Prepared, _run_forward
+    gen = torch.Generator(device="cuda").manual_seed(D)
+    q, k, v, w, b, g = (torch.randn((1, T, H, D), generator=gen, device="cuda") for _ in range(6))
+    f = torch.nn.functional
+    xs = [x.bfloat16() for x in (f.normalize(q, dim=-1), f.normalize(k, dim=-1), v,
+                                 torch.sigmoid(w), torch.sigmoid(b))] + [-f.softplus(g)]
+    p = _Prepared(*xs, D ** -0.5, None, 64)
+    out, hf, _, _ = _run_forward(p, flags=_lib.FWD_SAVE_A)
+    out_s, hf_s, _, _ = _run_forward(p, flags=_lib.FWD_SAVE_A | _lib.FWD_SEGMENTS(S))
+    assert torch.equal(out, out_s) and torch.equal(hf, hf_s)
