@@ -2181,6 +2181,43 @@ size_t bwd_ws_bytes(size_t nchunks, int BT, int D, size_t) {
 }
 
 
+// B1 over `units` (b,h) pairs or (head, sequence)s of NC chunks in all.  Where the
+// forward kept fragment tiles (scan_rows does not hold): the scan over fragments, the
+// transposed tiles in `kg` and `wt` ([NC][64][D] each, the DQG / DKG regions, which B3
+// writes afterwards).  Else bwd_state.
+template <typename T, int D>
+void launch_b1(hipStream_t st, size_t units, size_t NC, const BStateArgs<T>& sa, float* kg,
+               float* wt) {
+  constexpr int BT = 64;
+  if constexpr (sizeof(T) == 4) {
+    if (!scan_rows(4, units, D)) {
+      BScanArgs fa{};
+      fa.GL = sa.GL;
+      fa.DVPT = sa.DVPT;
+      fa.QDOT = sa.QDOT;
+      fa.dh_final = sa.dh_final;
+      fa.DHT = sa.DHT;
+      fa.DVNT = sa.DVNT;
+      fa.dh0 = sa.dh0;
+      fa.N = sa.N;
+      fa.units = (int)units;
+      fa.cu = sa.cu;
+      fa.S = sa.S;
+      fa.H = sa.H;
+      launch_bwd_scan<D>(st, NC, sa.W, sa.KgT, kg, wt, fa);
+      return;
+    }
+  }
+  constexpr int BW = 2;                       // column slices per scan workgroup
+  constexpr int BK = bstate_ksplit<T, D>();   // compute waves per column slice
+  // producer waves: four with the K-split (float32: the next chunk's DMA is bound
+  // by how fast it is issued), else two, which leaves the compute waves one per
+  // SIMD with 512 registers
+  constexpr int BP = BK > 1 ? 4 : 2;
+  hipLaunchKernelGGL((bwd_state<T, BT, D, BW, BP, BK>), dim3(units * (D / (16 * BW))),
+                     dim3(64 * (BW * BK + BP)), 0, st, sa);
+}
+
 // The backward at D = 256 (chunk 64): B2 by bwd_b2 (its tiles still fit LDS,
 // 136 KB), B3 by bwd_wy_wide (the D x D operands streamed in slices: the D = 128
 // kernel would need 266 KB), the reverse scan (single-buffered at this width) and
@@ -2213,34 +2250,8 @@ hipError_t launch_bwd_wide(hipStream_t st, int B, int T_len, int H, const void* 
   BStateArgs<T> sa{(const T*)(fws + F.W), (const T*)(fws + F.KgT),
                    reinterpret_cast<const float*>(fws + F.GL), buf(B_DVPT), buf(B_QDOT),
                    dh_final, N, buf(B_DHT), buf(B_DVNT), dh0, cu_chunks, cu_chunks ? nseq : 1, H};
-  constexpr int BW = 2, BK = bstate_ksplit<T, D>(), BP = BK > 1 ? 4 : 2;
-  const size_t units = cu_chunks ? (size_t)H * nseq : (size_t)B * H;
-  // B1: where the units leave CUs free, the scan over fragment tiles (the transposed
-  // tiles go into the DQG / DKG regions, which B3 writes afterwards); else bwd_state
-  bool frag = false;
-  if constexpr (sizeof(T) == 4) {
-    frag = !scan_rows(4, units, D);
-    if (frag) {
-      BScanArgs fa{};
-      fa.GL = sa.GL;
-      fa.DVPT = sa.DVPT;
-      fa.QDOT = sa.QDOT;
-      fa.dh_final = dh_final;
-      fa.DHT = sa.DHT;
-      fa.DVNT = sa.DVNT;
-      fa.dh0 = dh0;
-      fa.N = N;
-      fa.units = (int)units;
-      fa.cu = cu_chunks;
-      fa.S = sa.S;
-      fa.H = H;
-      launch_bwd_scan<D>(st, NC, (const float*)sa.W, (const float*)sa.KgT, buf(B_DQG), buf(B_DKG),
-                         fa);
-    }
-  }
-  if (!frag)
-    hipLaunchKernelGGL((bwd_state<T, BT, D, BW, BP, BK>), dim3(units * (D / (16 * BW))),
-                       dim3(64 * (BW * BK + BP)), 0, st, sa);
+  launch_b1<T, D>(st, cu_chunks ? (size_t)H * nseq : (size_t)B * H, NC, sa, buf(B_DQG),
+                  buf(B_DKG));
   launch_mark(st);
   if (NC > 0) {
     // B3 (gdn2_bwd.py:126-210): one fused kernel with the D x D operands streamed
@@ -2306,39 +2317,8 @@ hipError_t launch_bwd(hipStream_t st, int B, int T_len, int H, const void* q, co
     // variable-length batch (B = 1): one scan unit per (head, sequence)
     BStateArgs<T> sa{(const T*)fW, (const T*)fKgT, fGL, buf(B_DVPT), buf(B_QDOT), dh_final, N,
                      buf(B_DHT), buf(B_DVNT), dh0, cu_chunks, cu_chunks ? nseq : 1, H};
-    constexpr int BW = 2;                       // column slices per scan workgroup
-    constexpr int BK = bstate_ksplit<T, D>();   // compute waves per column slice
-    // producer waves: four with the K-split (float32: the next chunk's DMA is bound
-    // by how fast it is issued), else two, which leaves the compute waves one per
-    // SIMD with 512 registers
-    constexpr int BP = BK > 1 ? 4 : 2;
-    const size_t units = cu_chunks ? (size_t)H * nseq : (size_t)B * H;
-    // B1: where the units leave CUs free, the scan over fragment tiles (the transposed
-    // tiles go into the DQG / DKG regions, which B3 writes afterwards); else bwd_state
-    bool frag = false;
-    if constexpr (sizeof(T) == 4) {
-      frag = !scan_rows(4, units, D);
-      if (frag) {
-        BScanArgs fa{};
-        fa.GL = sa.GL;
-        fa.DVPT = sa.DVPT;
-        fa.QDOT = sa.QDOT;
-        fa.dh_final = dh_final;
-        fa.DHT = sa.DHT;
-        fa.DVNT = sa.DVNT;
-        fa.dh0 = dh0;
-        fa.N = N;
-        fa.units = (int)units;
-        fa.cu = cu_chunks;
-        fa.S = sa.S;
-        fa.H = H;
-        launch_bwd_scan<D>(st, NC, (const float*)sa.W, (const float*)sa.KgT, buf(B_DQG), buf(B_DKG),
-                           fa);
-      }
-    }
-    if (!frag)
-      hipLaunchKernelGGL((bwd_state<T, BT, D, BW, BP, BK>), dim3(units * (D / (16 * BW))),
-                         dim3(64 * (BW * BK + BP)), 0, st, sa);
+    launch_b1<T, D>(st, cu_chunks ? (size_t)H * nseq : (size_t)B * H, NC, sa, buf(B_DQG),
+                    buf(B_DKG));
     launch_mark(st);
     if (NC > 0) {
       // B3, one fused kernel
