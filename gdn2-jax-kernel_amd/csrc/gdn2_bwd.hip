@@ -2190,7 +2190,7 @@ void launch_b1(hipStream_t st, size_t units, size_t NC, const BStateArgs<T>& sa,
                float* wt) {
   constexpr int BT = 64;
   if constexpr (sizeof(T) == 4) {
-    if (!scan_rows(4, units, D)) {
+    if (!scan_rows(4, units, D, sa.N)) {
       BScanArgs fa{};
       fa.GL = sa.GL;
       fa.DVPT = sa.DVPT;

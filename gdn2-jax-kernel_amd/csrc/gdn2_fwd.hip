@@ -1187,7 +1187,7 @@ hipError_t launch_fwd(hipStream_t st, int B, int T_len, int H, const void* q, co
   // h^T / v_new^T tiles have no region (a variable-length workspace keeps them:
   // its size does not depend on flags)
   const bool fuse = fuse_ws && !a_dbg;
-  const bool rows = !fuse && scan_rows(sizeof(T), (size_t)B * H * (vl ? vl->nseq : 1), D);
+  const bool rows = !fuse && scan_rows(sizeof(T), (size_t)B * H * (vl ? vl->nseq : 1), D, N);
   const size_t seg_units = S_ws > 1 ? (size_t)B * H * S_ws : 0;
   const FwdLayout L = fwd_layout(NC, BT, D, sizeof(T), seg_units, !(flags & kFwdNoARegion),
                                  !fuse || vl != nullptr);

@@ -194,8 +194,13 @@ constexpr int scan_per_cu(int esize, int out_waves) {
 // shapes only, so that the backward knows what the forward kept.  At D = 128 on
 // 48 (b,h) of 128 chunks fwd_state takes 300 us and fwd_scan 368; on 24 of 32 75
 // and 44; at D = 256 on 12 of 64 405 and 175.
-constexpr bool scan_rows(int esize, size_t units, int D) {
-  return esize == 4 && units * (D / 16) > 256;
+// Also where one or two of the `chunks` per (b,h) (packed: in all) are too few for the
+// loads ahead of the steps to pay for the transposed fragments of the reverse scan:
+// forward and reverse scan of 2 (b,h) of one chunk at D = 64, 128, 256 9.3, 13.8 and
+// 19.0 us in rows, 13.0, 18.5 and 24.1 in fragments; of two 12.4, 19.0, 29.7 and
+// 14.9, 21.2, 28.7; of four 18.6, 28.9, 50.1 and 18.0, 26.5, 38.1.
+constexpr bool scan_rows(int esize, size_t units, int D, long long chunks) {
+  return esize == 4 && (units * (D / 16) > 256 || chunks <= 2);
 }
 
 // Segments of the forward state scan for BH (b,h) pairs of N chunks with

@@ -284,11 +284,11 @@ def _residual_views(p: _Prepared, ws: torch.Tensor):
     # bfloat16 HT, VnT keep their last dimension in chained order (gdn2_common.h
     # kpos).  W (negated), UT and KgT are in operand-fragment order (float32 W and
     # KgT as hi and lo fragments, UT in fragments of 16 tokens), except float32
-    # tiles where the units fill the device (scan_rows in gdn2_layout.h): rows, W
-    # and KgT in the split pair layout.  Undo all of it.
+    # tiles where the units fill the device or have one or two chunks (scan_rows in
+    # gdn2_layout.h): rows, W and KgT in the split pair layout.  Undo all of it.
     chained = p.tile_dt == torch.bfloat16
     nat = lambda x, n: x[..., _kpos_index(n, x.device)] if chained else x
-    rows = not chained and B * H * (D // 16) > 256
+    rows = not chained and (B * H * (D // 16) > 256 or N <= 2)
     spl = _frag_decode if chained else _split_decode if rows else _split_frag_decode
     tile = _frag_decode if chained else (lambda x: x) if rows else _frag16_decode
     return {

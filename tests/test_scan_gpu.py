@@ -75,6 +75,26 @@ def test_training_scan_edges(D, chunks, short, full):
         assert torch.all((a.double() - r).abs() <= 1e-4 + 1e-4 * r.abs()), name
 
 
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("chunks,H", [(2, 3), (3, 3), (3, None)])
+def test_kept_tiles_of_both_layouts(D, chunks, H):
+    """The float32 tiles that a residual-keeping forward leaves, on both sides of each
+    line of the layout rule (rows for up to two chunks and for a full device, else
+    fragments), against the oracle's restatement of the reference's kernels."""
+    import gdn2_package as gp
+    H = H or 256 // (D // 16) + 1
+    xs = O.make_inputs(1, chunks * 64, H, D, seed=chunks + D)
+    h0 = (0.1 * np.random.default_rng(2).standard_normal((1, H, D, D))).astype(np.float32)
+    dev = torch.device("cuda")
+    _, _, res = gp.gdn2_pallas_forward_with_residuals(
+        *[torch.tensor(x, device=dev) for x in xs], D ** -0.5, h0=torch.tensor(h0, device=dev),
+        chunk_size=64)
+    _, _, ref = O.chunked_fwd(*xs, D ** -0.5, h0=h0, BT=64, clip=False, return_residuals=True)
+    for key in ["w_pseudo", "u", "kg", "qg", "gc_last", "h_pre_all", "v_new_all"]:
+        # 1e-4 as test_fwd_gpu.py's intermediates
+        assert np.allclose(res[key].cpu().numpy(), ref[key], rtol=1e-4, atol=1e-4), key
+
+
 @pytest.mark.parametrize("dtype,D,BT,H,S,save", [
     # more than 256 16-column slices in the final pass, with and without kept residuals
     (torch.float32, 64, 64, 9, 8, False), (torch.float32, 64, 64, 9, 8, True),
@@ -114,7 +134,10 @@ def test_segments_of_a_full_device(dtype, D, BT, H, S, save):
 
 
 @pytest.mark.parametrize("D,H,seqs", [(64, 5, 12), (64, 5, 13), (128, 3, 10), (128, 3, 11),
-                                      (256, 1, 16), (256, 1, 17)])
+                                      (256, 1, 16), (256, 1, 17),
+                                      # one, two and four chunks in all
+                                      (128, 3, 2), (64, 5, 3), (128, 3, 3), (256, 1, 3),
+                                      (128, 3, 4)])
 def test_packed_training_layouts(D, H, seqs):
     """Packed training with (head, sequence) counts on both sides of the rule that lays
     the float32 tiles out, which the forward and the backward apply separately: every
