@@ -305,8 +305,15 @@ def pmc_train_run():
     print(json.dumps({"pmc_train_run": 1, "copy_bytes": COPY_BYTES}), flush=True)
 
 
+# the training step's kernels at its shape, and every kernel that a counter run can name
 TRAIN_KERNELS = ("fwd_prep", "fwd_state", "fwd_out", "bwd_b2", "bwd_state", "bwd_wy",
                  "gram_bwd")
+KERNEL_NAMES = TRAIN_KERNELS + ("fwd_scan", "bwd_scan", "frag_transpose", "seg_combine",
+                                "decode_step")
+
+
+def _short_name(name):
+    return next((k for k in KERNEL_NAMES if k in name), name)
 
 
 def train_traffic_from(fetch_dir, write_dir):
@@ -320,8 +327,7 @@ def train_traffic_from(fetch_dir, write_dir):
     bf16 = lambda n: "DF16b" in n or "__bf16" in n or "bfloat16" in n
     rows = {}
     for k in TRAIN_KERNELS:
-        names = [n for n in fetch if k in n and "gdn2" in n and not bf16(n)
-                 and not (k == "fwd_state" and "seg_" in n)]
+        names = [n for n in fetch if k in n and "gdn2" in n and not bf16(n)]
         if len(names) != 1:
             raise SystemExit(f"{k}: expected one float32 kernel, found {names}")
         n = names[0]
@@ -360,9 +366,7 @@ def mfma_from(run_dir):
     for (_, name), d in sorted(per.items()):
         if "gdn2" not in name:
             continue
-        short = next((k for k in ("fwd_prep", "fwd_scan", "fwd_state", "fwd_out", "bwd_b2",
-                                  "bwd_scan", "bwd_state", "bwd_wy", "gram_bwd") if k in name),
-                     name)
+        short = _short_name(name)
         dt = "bf16" if ("DF16b" in name or "__bf16" in name or "bool" in name) else "fp32"
         f32 = 512 * d.get("SQ_INSTS_VALU_MFMA_MOPS_F32", 0)
         b16 = 512 * d.get("SQ_INSTS_VALU_MFMA_MOPS_BF16", 0)
@@ -405,8 +409,7 @@ def sq_from(run_dirs):
             rows = [r for r in csv.DictReader(fh) if "gdn2" in r["Kernel_Name"]]
 
         def key_of(name):
-            short = next((k for k in TRAIN_KERNELS if k in name), name)
-            return f"{short} ({'bf16' if ('DF16b' in name or '__bf16' in name) else 'fp32'})"
+            return f"{_short_name(name)} ({'bf16' if ('DF16b' in name or '__bf16' in name) else 'fp32'})"
         last = {}
         for r in rows:
             k = key_of(r["Kernel_Name"])

@@ -32,7 +32,7 @@ def write_run(d: Path, rows):
                         "End_Timestamp": 1000 + ns})
 
 
-F32 = "void gdn2::fwd_state<float, 64, 128, 2, 4, 2, 0>(gdn2::StateArgs<float>)"
+F32 = "void gdn2::fwd_state<64, 128, false>(gdn2::ScanArgs<float>)"
 BF = "void gdn2::fwd_prep<__bf16, float, 128, 128, __bf16, 0>(gdn2::PrepArgs<__bf16>)"
 
 
@@ -78,6 +78,21 @@ def test_sq_from_takes_last_dispatch_and_merges_passes(tmp_path, capsys):
     assert r["active_valu"] == pytest.approx(40 / 400)
     assert r["valu_per_wave"] == 100 and r["lds_per_wave"] == 2
     assert r["lds_bank_conflict_per_wave"] == 3 and r["waves"] == 4
+
+
+@pytest.mark.parametrize("kernel,key", [
+    # as the profiler prints the built kernels
+    ("void gdn2::fwd_scan<float, 64, 128, 2, 1, 0, false>(gdn2::ScanArgs<float>)",
+     "fwd_scan (fp32)"),
+    ("_ZN4gdn28fwd_scanIDF16bLi128ELi128ELi1ELi2ELi1ELb0EEEvNS_8ScanArgsIT_EE", "fwd_scan (bf16)"),
+    ("void gdn2::bwd_scan<64, 128, 2>(gdn2::BScanArgs)", "bwd_scan (fp32)"),
+    ("void gdn2::frag_transpose<64, 128>(float const*, float*, float const*, float*, int)",
+     "frag_transpose (fp32)")])
+def test_reducers_name_the_scan_kernels(tmp_path, capsys, kernel, key):
+    write_run(tmp_path, [(1, kernel, "SQ_WAVES", 2.0, 10), (1, kernel, "SQ_WAVE_CYCLES", 8.0, 10)])
+    assert list(bench.sq_from([tmp_path])) == [key]
+    assert list(bench.mfma_from(tmp_path)) == [key]
+    capsys.readouterr()
 
 
 def test_counter_means_refuse_two_runs_in_one_directory(tmp_path):
