@@ -17,9 +17,10 @@
 // workgroups -- on different XCDs -- fetch and write back each line.  With 16, 32
 // and 64 columns (bfloat16 tokens, D = 128, state updated in place, kernels back to
 // back): 32 x 6 (b,h) 11.7, 6.2 and 6.1 us, 128 x 6 28.9, 19.4 and 16.6, 512 x 6
-// 95.9, 64.1 and 61.2 us (403 MB: 4.2, 6.3 and 6.6 TB/s); 8 x 6 at D = 256 10.7,
-// 6.4 and 6.6 us; 2 at D = 64 3.45, 3.75 and 4.40 us.  So: 64 columns from 512 such
-// workgroups on (two per CU), 16 where 32 would leave fewer than 32 workgroups.
+// 95.9, 64.1 and 61.2 us (403 MB, of which the 201 MB state stays in the 256 MB cache;
+// written to a new state 78 us, the rate of a copy); 8 x 6 at D = 256 10.7, 6.4 and
+// 6.6 us; 2 at D = 64 3.45, 3.75 and 4.40 us.  So: 64 columns from 512 such workgroups
+// on (two per CU), 16 where 32 would leave fewer than 32 workgroups.
 #include "gdn2_common.h"
 
 namespace gdn2 {

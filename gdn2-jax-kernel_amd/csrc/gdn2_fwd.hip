@@ -4,7 +4,7 @@
 //             gdn2_fwd.py:99-139, 174-243, 264-295
 //   fwd_scan  (one workgroup per (b,h) and 16 or 32 value columns, serial over
 //             chunks; gdn2_scan.h) the state half of kernel D, gdn2_fwd.py:347-358;
-//             float32 residuals on a full device: fwd_state
+//             float32 tiles in rows (scan_rows): fwd_state
 //   fwd_out   (one workgroup per chunk)      the output half of kernel D,
 //             gdn2_fwd.py:349-353
 //

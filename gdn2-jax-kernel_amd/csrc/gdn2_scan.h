@@ -685,10 +685,10 @@ __global__ void __launch_bounds__(64 * (KS + NO + 1), scan_per_cu(sizeof(T), NO)
 
 // ---------------------------------------------------------------------------
 // The scan of float32 tiles in rows (scan_rows in gdn2_layout.h), where the units
-// fill the device: one workgroup per unit and 32 value columns, which shares each
-// tile through LDS -- two 16-column slices with two K-split compute waves each
-// (half of h's rows) and four producer waves.  W and kg^T come in the split pair
-// layout (gdn2_common.h), u^T in rows.
+// fill the device or have one or two chunks: one workgroup per unit and 32 value
+// columns, which shares each tile through LDS -- two 16-column slices with two
+// K-split compute waves each (half of h's rows) and four producer waves.  W and kg^T
+// come in the split pair layout (gdn2_common.h), u^T in rows.
 //
 // While the compute waves work on chunk c, the producers stream chunk c+1 (W,
 // kg^T, g_last and this workgroup's u^T rows) into LDS with

@@ -2,7 +2,7 @@
 reference README does (fwd.CLIP = 1e3, README.md:87-92): every stage sanitize
 of the library then saturates at the new bound.  Each kernel unit holds its own
 copy of the bound (gdn2_set_clip sets them all), so each is checked here through
-a path that runs it: the forward (fwd_prep / fwd_state / fwd_out), the training
+a path that runs it: the forward (fwd_prep / the state scan / fwd_out), the training
 backward (bwd_b2 / bwd_state / bwd_wy / gram_bwd), the decode step and a stage
 function (reverse cumsum).  Against the oracle with the same CLIP (its sanitize
 reads the module constant at call time), on the saturation scale: |got - ref| <=
